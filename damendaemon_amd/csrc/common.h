@@ -158,3 +158,4 @@ DD_DEV float xor32_sum(float x) {
   } while (0)
 
 static inline long dd_cdiv(long a, long b) { return (a + b - 1) / b; }
+static inline bool dd_aligned(const void *p, unsigned bytes) { return ((uintptr_t)p & (bytes - 1)) == 0; }

@@ -177,6 +177,43 @@ __global__ __launch_bounds__(256) void store_pages_q8_kernel(const void *key, co
   vs[row * ng + gi] = q8_group<DT>(value, src, group, cv + dst);
 }
 
+// The same with eight channels per lane and 2^shift lanes per group (q8.h):
+// lane i of n = (tokens * kv_heads * groups) << shift.
+template <int DT>
+__global__ __launch_bounds__(256) void store_pages_q8_lanes_kernel(const void *key, const void *value,
+                                                                   const int64_t *slot_map, unsigned n,
+                                                                   unsigned per_token, int kv_heads, int dim,
+                                                                   int group, int shift, int page, long capacity,
+                                                                   signed char *ck, signed char *cv,
+                                                                   unsigned short *ks, unsigned short *vs) {
+  const unsigned i = blockIdx.x * 256u + threadIdx.x;
+  const unsigned g = i >> shift;
+  const int c = 8 * (int)(i & ((1u << shift) - 1));
+  const unsigned ng = (unsigned)(dim / group);
+  const unsigned t = g / per_token, rem = g - t * per_token;
+  const unsigned kh = rem / ng, gi = rem - kh * ng;
+  const bool in = i < n && c < group;
+  const long s = in ? slot_map[t] : -1;
+  const long phys = s < 0 ? -1 : s <= 0x7fffffffL ? (long)((unsigned)s / (unsigned)page) : s / page;
+  const bool on = s >= 0 && phys < capacity;
+  const long src = (long)g * group + c;      // (token, KV head, group) rows are contiguous
+  float k[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (in) {
+    q8_load8<DT>(key, src, k);
+    q8_load8<DT>(value, src, v);
+  }
+  unsigned short kbits, vbits;
+  const u32x2 kq = q8_lanes(k, shift, &kbits), vq = q8_lanes(v, shift, &vbits);
+  if (!on) return;
+  const long row = (phys * kv_heads + kh) * page + (s - phys * page);
+  *(u32x2 *)(ck + row * dim + gi * group + c) = kq;
+  *(u32x2 *)(cv + row * dim + gi * group + c) = vq;
+  if (c == 0) {
+    ks[row * ng + gi] = kbits;
+    vs[row * ng + gi] = vbits;
+  }
+}
+
 }  // namespace
 
 extern "C" int dd_pack_batch(const int64_t *lengths, const int64_t *starts, const int64_t *slots, int n,
@@ -233,12 +270,32 @@ extern "C" int dd_store_kv_pages_q8(const void *key, const void *value, int dtyp
     return DD_EINVAL;
   const long work = (long)tokens * kv_heads * (dim / group);
   if (work == 0) return DD_OK;
-  const dim3 grid((unsigned)dd_cdiv(work, 256));
   hipStream_t s = (hipStream_t)stream;
   auto *ck = (signed char *)cache_k;
   auto *cv = (signed char *)cache_v;
   auto *ks = (unsigned short *)k_scale;
   auto *vs = (unsigned short *)v_scale;
+  // eight channels per lane where rows start on 16 bytes and the lanes fit 32 bits
+  const int shift = q8_lane_shift(group);
+  if (shift >= 0 && (work << shift) <= 0x7fffffffL && dd_aligned(key, 16) && dd_aligned(value, 16) &&
+      dd_aligned(cache_k, 8) && dd_aligned(cache_v, 8)) {
+    const unsigned n = (unsigned)(work << shift);
+    const dim3 lanes((unsigned)dd_cdiv(n, 256));
+#define DD_Q8_LANES(DT)                                                                                          \
+  hipLaunchKernelGGL(store_pages_q8_lanes_kernel<DT>, lanes, dim3(256), 0, s, key, value, slot_map, n,           \
+                     (unsigned)(kv_heads * (dim / group)), kv_heads, dim, group, shift, page_size, (long)capacity, \
+                     ck, cv, ks, vs)
+    switch (dtype) {
+      case DD_F32: DD_Q8_LANES(DD_F32); break;
+      case DD_F16: DD_Q8_LANES(DD_F16); break;
+      case DD_BF16: DD_Q8_LANES(DD_BF16); break;
+      default: return DD_EUNSUPPORTED;
+    }
+#undef DD_Q8_LANES
+    DD_LAUNCH_CHECK();
+    return DD_OK;
+  }
+  const dim3 grid((unsigned)dd_cdiv(work, 256));
 #define DD_Q8_STORE(DT)                                                                                    \
   hipLaunchKernelGGL(store_pages_q8_kernel<DT>, grid, dim3(256), 0, s, key, value, slot_map, (long)tokens, \
                      kv_heads, dim, group, page_size, (long)capacity, ck, cv, ks, vs)

@@ -330,7 +330,7 @@ extern "C" int dd_rope_batch(const void *qkv, int qkv_dtype, const void *cos, co
   p.eps = eps;
   hipStream_t s = (hipStream_t)stream;
   // the 16-byte accesses of the vector kernel need 16-byte aligned rows
-  auto a16 = [](const void *q) { return ((uintptr_t)q & 15) == 0; };
+  auto a16 = [](const void *q) { return dd_aligned(q, 16); };
   const bool aligned = a16(qkv) && a16(cos) && a16(sin) && a16(query) && a16(cache_k) && a16(cache_v) &&
                        a16(key_out) && a16(value_out);
   if (aligned && rotary_dim == dim && (dim == 64 || dim == 128 || dim == 256) && cache_dtype == qkv_dtype) {
