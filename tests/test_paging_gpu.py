@@ -292,3 +292,35 @@ def test_rope_partial_rotary_fp32():
     q = kernels.rope_batch(qkv.to(DEV), cos.to(DEV), sin.to(DEV), pos.to(DEV), slots.to(DEV), dk, dv, heads)
     eq, eck, ecv, _, _ = O.rope_batch(qkv, cos, sin, pos, slots, ck, cv, heads)
     assert torch.equal(q.cpu(), eq) and torch.equal(dk.cpu(), eck) and torch.equal(dv.cpu(), ecv)
+
+
+@pytest.mark.parametrize('dim,rd', [(8, 8), (16, 16), (24, 16), (40, 32), (72, 64), (80, 80), (80, 40), (96, 48), (160, 160),
+                                    (256, 64), (512, 512), (520, 16)])
+@pytest.mark.parametrize('dtype,precise', [(torch.float32, True), (torch.float32, False), (torch.bfloat16, False)])
+def test_rope_lane_layouts(dim, rd, dtype, precise):
+    """Head sizes and rotary widths at and off the vector kernel's lane groups, few tokens (one
+    workgroup per pass over the heads) and more than 256 (one per token), pages of 24 tokens,
+    unmapped and out-of-range slots; bit-exact, dense copies included."""
+    g = torch.Generator().manual_seed(dim + rd)
+    heads, kh, page, cap, context = 5, 3, 24, 30, 700
+    for tokens in (3, 257):
+        pos = torch.randperm(context, generator=g)[:tokens]
+        slots = torch.randint(0, 2, (tokens,), generator=g)
+        slots[1] = 2                                  # past the table: no cache row
+        table = torch.full((2, 30), -1, dtype=torch.int32)
+        table.view(-1)[torch.randperm(60, generator=g)[:cap]] = torch.randperm(cap, generator=g).to(torch.int32)
+        qkv = torch.randn((tokens, (heads + 2 * kh) * dim), generator=g).to(dtype)
+        cos, sin = torch.randn((context, rd), generator=g), torch.randn((context, rd), generator=g)
+        ck = torch.zeros((cap, kh, page, dim), dtype=dtype)
+        cv = torch.zeros_like(ck)
+        dk, dv = ck.to(DEV), cv.to(DEV)
+        q, k, v = kernels.rope_batch(qkv.to(DEV), cos.to(DEV), sin.to(DEV), pos.to(DEV), slots.to(DEV), dk, dv, heads,
+                                     precise=precise, page_table=table.to(DEV), materialize=True)
+        # the oracle writes unmapped rows into one more page, which is dropped
+        wide = torch.cat((table, torch.full((1, 30), -1, dtype=torch.int32)))
+        wide[wide < 0] = cap
+        spare = torch.zeros((cap + 1, kh, page, dim), dtype=dtype)
+        eq, eck, ecv, ek, ev = O.rope_batch(qkv, cos, sin, pos, slots, spare, spare, heads, precise=precise,
+                                            page_table=wide)
+        for have, want in ((q, eq), (k, ek), (v, ev), (dk, eck[:cap]), (dv, ecv[:cap])):
+            assert torch.equal(have.cpu(), want)
