@@ -48,6 +48,9 @@ SIGNATURES['dd_prefill_attention'] = [_p, _p, _p, _i, _p, _p, _p, _i, _i, _i, _p
                                       _f, _p, _i, _p, _p, _p]
 SIGNATURES['dd_prefill_flag_count'] = [_i, _i, _i, _i, _i, _i]
 SIGNATURES['dd_prefill_attention_phase'] = SIGNATURES['dd_prefill_attention'][:-1] + [_i, _p]
+SIGNATURES['dd_prefill_attention_split'] = SIGNATURES['dd_prefill_attention'][:-1] + [_i, _i, _p, _i64, _i, _p]
+SIGNATURES['dd_prefill_split'] = [_p, _p, _i, _i, _i, _i, _i, _i, _i, ctypes.POINTER(_i), ctypes.POINTER(_i),
+                                  ctypes.POINTER(_i64)]
 SIGNATURES['dd_prefill_plan'] = [_p, _p, _p, _i, _i, _i, _i, _i, _i, _p, _i]
 SIGNATURES['dd_prefill_geometry'] = [_i, ctypes.POINTER(_i), ctypes.POINTER(_i)]
 SIGNATURES['dd_prefill_indices'] = [_i64, _i, _i, _i64, _i64, _p, _p]
@@ -102,6 +105,13 @@ def require_device(*tensors):
                              '(there is no CPU path)')
 
 
+def refuse_capture():
+    """Calls whose launches depend on host copies of the segments are prepared outside a graph capture."""
+    if torch.cuda.is_current_stream_capturing():
+        raise RuntimeError('host upload during HIP graph capture: prepare the call (prepare_prefill, '
+                           'pack_batch) before capturing and capture only the launch')
+
+
 class _Staging:
     """Pinned host buffers for the small per-call uploads (segment metadata,
     prefill plans), reused round-robin instead of pinning fresh memory on
@@ -123,9 +133,7 @@ class _Staging:
         on the current stream; returns the device tensor.  Not under graph
         capture: a replay would copy whatever the reused pinned slot holds by
         then (prepare the call outside the capture and capture its run())."""
-        if torch.cuda.is_current_stream_capturing():
-            raise RuntimeError('host upload during HIP graph capture: prepare the call (prepare_prefill, '
-                               'pack_batch) before capturing and capture only the launch')
+        refuse_capture()
         host = host.contiguous()
         with self._lock:
             return self._upload(host, torch.device(device))

@@ -65,7 +65,8 @@ static int prefill_entry(int phase, const void *q, const void *k, const void *v,
                          const int64_t *cu_seqlens, const int64_t *context_lens, const int64_t *slots, int n,
                          int max_len, int max_context, const int32_t *page_table, int table_rows, int table_width,
                          int heads, int kv_heads, int dim, int page_size, int64_t capacity, int window, float scale,
-                         const int32_t *plan, int plan_len, int32_t *flags, void *out, void *stream) {
+                         const int32_t *plan, int plan_len, int32_t *flags, void *out, void *stream,
+                         int split_tiles = 0, int max_splits = 1, float *part = nullptr, int64_t part_floats = 0) {
   if (phase < 1 || phase > 3) return DD_EINVAL;
   if (!q || !k || !v || !cu_seqlens || !context_lens || !slots || !page_table || !out || n < 0 || max_len < 0 ||
       heads <= 0 || kv_heads <= 0 || heads % kv_heads || page_size <= 0 || capacity <= 0 || table_width <= 0)
@@ -139,6 +140,15 @@ static int prefill_entry(int phase, const void *q, const void *k, const void *v,
   p.scale_log2 = __builtin_fabsf(scale) * kLog2e;
   p.q_sign = scale < 0.f ? 0x80008000u : 0u;
   p.flags = needs_flags > 0 ? flags : nullptr;
+  p.max_splits = 1;
+  if (max_splits > 1) {
+    if (split_tiles < 1 || plan) return DD_EINVAL;
+    const long items = (long)n * kv_heads * dd_cdiv(max_len, geom.cols / p.G);
+    if (!part || (long)part_floats / prefill_part_floats(geom.cols, dim) / max_splits < items) return DD_ESCRATCH;
+    p.split_tiles = split_tiles;
+    p.max_splits = max_splits;
+    p.part = part;
+  }
   int rc = DD_OK;
   if (phase & 1) {
     rc = DD_EUNSUPPORTED;
@@ -174,6 +184,93 @@ extern "C" int dd_prefill_attention_phase(const void *q, const void *k, const vo
   return prefill_entry(phase, q, k, v, dtype, cu_seqlens, context_lens, slots, n, max_len, max_context, page_table,
                        table_rows, table_width, heads, kv_heads, dim, page_size, capacity, window, scale, plan,
                        plan_len, flags, out, stream);
+}
+
+extern "C" int dd_prefill_attention_split(const void *q, const void *k, const void *v, int dtype,
+                                          const int64_t *cu_seqlens, const int64_t *context_lens,
+                                          const int64_t *slots, int n, int max_len, int max_context,
+                                          const int32_t *page_table, int table_rows, int table_width, int heads,
+                                          int kv_heads, int dim, int page_size, int64_t capacity, int window,
+                                          float scale, const int32_t *plan, int plan_len, int32_t *flags, void *out,
+                                          int split_tiles, int max_splits, float *scratch, int64_t scratch_floats,
+                                          int phase, void *stream) {
+  return prefill_entry(phase, q, k, v, dtype, cu_seqlens, context_lens, slots, n, max_len, max_context, page_table,
+                       table_rows, table_width, heads, kv_heads, dim, page_size, capacity, window, scale, plan,
+                       plan_len, flags, out, stream, split_tiles, max_splits, scratch, scratch_floats);
+}
+
+// Whether a call needs no plan, and how its key tiles are split: see the
+// header.  A work item (256 or 128 query columns, all its keys) is a long
+// serial chain, and a call with fewer items than CUs leaves the rest idle: a
+// 333-token chunk on 5,000 keys with 4 KV heads is 40 items of 84 tiles.  The
+// keys are then split into equal shares of whole tiles, as few tiles each as
+// keep the units of the whole call at one per CU (one workgroup fits per CU).
+// A split costs its workgroup's prologue and epilogue again (about five
+// tiles' time) and the call a merge launch, so shares are at least four
+// tiles, and nothing is split that would not get four tiles shorter.
+// (That chunk, fp16, 28 heads of 128: 141 us on 40 workgroups, 42 us on 240
+// and 7 us of merge.)
+extern "C" int dd_prefill_split(const int64_t *lengths, const int64_t *starts, int n, int heads, int kv_heads,
+                                int dim, int dtype, int window, int workgroups, int *split_tiles, int *max_splits,
+                                int64_t *scratch_floats) {
+  if (!lengths || !starts || n < 0 || heads <= 0 || kv_heads <= 0 || heads % kv_heads || !split_tiles || !max_splits ||
+      !scratch_floats)
+    return DD_EINVAL;
+  *split_tiles = 0;
+  *max_splits = 1;
+  *scratch_floats = 0;
+  Geometry g;
+  if (dtype == DD_F32 || !geometry(dim, &g) || g.cols < heads / kv_heads) return DD_EUNSUPPORTED;
+  const int rows = g.cols / (heads / kv_heads);
+  long items = 0, max_tiles = 0;
+  for (int i = 0; i < n; ++i) {
+    if (lengths[i] < 0 || starts[i] < 0 || lengths[i] + starts[i] > 0x7fffffffL) return DD_EINVAL;
+    items += dd_cdiv(lengths[i], rows);
+    max_tiles = std::max<long>(max_tiles, dd_cdiv(lengths[i], rows));
+  }
+  items *= kv_heads;
+  const long grid_items = (long)n * kv_heads * max_tiles;
+  if (grid_items > 0x7fffffffL) return DD_EUNSUPPORTED;
+  if (items > workgroups) return DD_EUNSUPPORTED;   // enough items: dd_prefill_plan's schedule
+  // units of the call with shares of `share` tiles; the longest item's tiles and all items'
+  long longest = 0, total = 0;
+  auto units = [&](long share) {
+    long count = 0;
+    total = 0;
+    for (int i = 0; i < n; ++i)
+      for (long r0 = 0; r0 < lengths[i]; r0 += rows) {
+        const long k_hi = starts[i] + std::min<long>(lengths[i], r0 + rows);
+        const long k_lo = window > 0 ? std::max<long>(0, starts[i] + r0 - window + 1) : 0;
+        const long tiles = (k_hi - 1) / g.kt - k_lo / g.kt + 1;
+        longest = std::max(longest, tiles);
+        total += tiles;
+        count += dd_cdiv(tiles, share);
+      }
+    total *= kv_heads;
+    return count * kv_heads;
+  };
+  constexpr long kLeast = 4, kGain = 4;
+  (void)units(kLeast);
+  const long per = prefill_part_floats(g.cols, dim) * grid_items;
+  // the grid and the scratch are those of the longest item for all: at most 1 GiB
+  const long most = per > 0 ? std::max(1L, (1L << 28) / per) : 1;
+  long share = longest;
+  long lo = kLeast, hi = longest;   // (one share per item always fits)
+  while (lo < hi) {
+    const long mid = (lo + hi) / 2;
+    if (units(mid) <= workgroups) hi = mid; else lo = mid + 1;
+  }
+  if (longest - lo >= kGain) {
+    // (equal shares of the longest item where they keep to the units above)
+    const long splits = std::min(dd_cdiv(longest, lo), most);
+    const long even = std::max(kLeast, dd_cdiv(longest, splits));
+    share = units(even) <= workgroups ? even : lo;
+  }
+  if (share >= longest) return DD_OK;
+  *split_tiles = (int)share;
+  *max_splits = (int)dd_cdiv(longest, share);
+  *scratch_floats = per * *max_splits;
+  return DD_OK;
 }
 
 extern "C" int dd_prefill_flag_count(int n, int max_len, int heads, int kv_heads, int dim, int dtype) {

@@ -35,6 +35,11 @@ struct PrefillParams {
   float scale_log2;     // |scale| * log2(e)
   unsigned q_sign;      // 0x80008000 when scale < 0: q enters negated (exact), so logits use |scale|
   int32_t *flags;       // bf16 pages, D 64/128: per work item, 1 = result must be recomputed exactly
+  // Without a plan, a work item's key tiles may be split over max_splits
+  // workgroups of split_tiles tiles each (max_splits 1: not split), whose
+  // partial results go to `part` and are combined by prefill_merge_kernel.
+  int split_tiles, max_splits;
+  float *part;
 };
 
 // One work item of the prefill kernels: query tile qt of group grp =
@@ -43,18 +48,29 @@ struct PrefillParams {
 // workgroup reads them with one load instead of a chain of two.
 constexpr int kPlanInts = DD_PREFILL_PLAN_INTS;   // item, tok0, len, start, slot, rounds, 2 unused
 struct PrefillItem {
-  int grp, qt, seg, len, start;
+  int grp, qt, seg, len, start, split;
   long tok0, slot;
 };
+DD_DEV void prefill_segment(const PrefillParams &p, PrefillItem &it) {
+  it.seg = it.grp / p.KH;
+  it.tok0 = p.cu[it.seg];
+  it.len = (int)(p.cu[it.seg + 1] - it.tok0);
+  it.start = (int)p.ctx[it.seg] - it.len;
+  it.slot = p.slots[it.seg];
+}
 // Work items per workgroup under a plan: the plan holds `rounds` entries per
 // workgroup, round-major (entry round * gridDim.x + blockIdx.x); every entry
-// stores the count (field 5).  1 without a plan.
-DD_DEV int prefill_rounds(const PrefillParams &p) {
-  return p.plan ? p.plan[(long)kPlanInts * blockIdx.x + 5] : 1;
-}
-// Item of round `round` of this workgroup; false: nothing to do
-DD_DEV bool prefill_item(const PrefillParams &p, PrefillItem &it, int round = 0) {
-  if (p.plan) {
+// stores the count (field 5).
+DD_DEV int prefill_rounds(const PrefillParams &p) { return p.plan[(long)kPlanInts * blockIdx.x + 5]; }
+// Item of round `round` of this workgroup; false: nothing to do.  Without a
+// plan the units (group, split, query tile), query tiles innermost and
+// longest first, are cut into 8 runs of equal length, one per XCD
+// (consecutive workgroups go to the 8 XCDs round-robin, each with its own
+// L2), so that the query tiles that read the same keys share an L2 and no XCD
+// gets more workgroups than another.
+template <bool PLAN>
+DD_DEV bool prefill_item(const PrefillParams &p, PrefillItem &it, int round) {
+  if constexpr (PLAN) {
     const int32_t *e = p.plan + (long)kPlanInts * ((long)round * gridDim.x + blockIdx.x);
     const int item = e[0];
     if (item < 0) return false;
@@ -65,22 +81,38 @@ DD_DEV bool prefill_item(const PrefillParams &p, PrefillItem &it, int round = 0)
     it.len = e[2];
     it.start = e[3];
     it.slot = e[4];
+    it.split = 0;
     return it.grp < p.n * p.KH;
+  } else {
+    const int units = p.n * p.KH * p.max_splits * p.max_tiles;
+    const int per_xcd = (units + 7) / 8;
+    const int j = blockIdx.x >> 3;
+    const int u = (int)(blockIdx.x & 7) * per_xcd + j;
+    if (j >= per_xcd || u >= units) return false;
+    const int gs = u / p.max_tiles;
+    it.grp = gs / p.max_splits;
+    it.split = gs - it.grp * p.max_splits;
+    it.qt = p.max_tiles - 1 - (u - gs * p.max_tiles);
+    prefill_segment(p, it);
+    return true;
   }
-  // Without a plan: consecutive workgroups go to the 8 XCDs round-robin,
-  // each XCD with its own L2; every query tile of one (segment, KV head)
-  // group is sent to the same XCD, longest first.
-  const int xcd = blockIdx.x & 7;
-  const int j = blockIdx.x >> 3;
-  it.grp = xcd + 8 * (j / p.max_tiles);
-  it.qt = p.max_tiles - 1 - j % p.max_tiles;
-  if (it.grp >= p.n * p.KH) return false;
-  it.seg = it.grp / p.KH;
-  it.tok0 = p.cu[it.seg];
-  it.len = (int)(p.cu[it.seg + 1] - it.tok0);
-  it.start = (int)p.ctx[it.seg] - it.len;
-  it.slot = p.slots[it.seg];
-  return true;
+}
+
+// Key tiles kt_first .. kt_last of a work item of query rows r0 .. + rows_here,
+// narrowed to its split's share; the number of splits the item has (its last
+// split, should the caller's max_splits be too small for it, takes the rest).
+template <bool SPLIT>
+DD_DEV int prefill_tiles(const PrefillParams &p, const PrefillItem &it, int kt, int r0, int rows_here, int &kt_first,
+                         int &kt_last) {
+  const int k_hi = it.start + r0 + rows_here;  // exclusive
+  const int k_lo = p.window > 0 ? max(0, it.start + r0 - p.window + 1) : 0;
+  kt_first = k_lo / kt;
+  kt_last = (k_hi - 1) / kt;
+  if (!SPLIT) return 1;
+  const int nsplit = min((kt_last - kt_first) / p.split_tiles + 1, p.max_splits);
+  kt_first += it.split * p.split_tiles;
+  if (it.split + 1 < nsplit) kt_last = kt_first + p.split_tiles - 1;
+  return nsplit;
 }
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -95,6 +127,13 @@ DD_DEV unsigned pack2(float a, float b) {
   } else {
     return (unsigned)float_to_f16_bits(a) | ((unsigned)float_to_f16_bits(b) << 16);
   }
+}
+
+// Floats of one split's partial result: per wave of `columns` / 32, 32 columns
+// of O^T over whole 32-dim blocks, in accumulator order ((dim block, register
+// quad), lane), then the 32 running offsets and the 32 denominators.
+constexpr long prefill_part_floats(int columns, int dim) {
+  return (long)(columns / 32) * (32L * ((dim + 31) / 32 * 32) + 64);
 }
 
 // 32-bit word 3 of a raw (untyped) buffer resource.

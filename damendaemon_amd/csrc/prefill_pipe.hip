@@ -64,8 +64,9 @@
 //     (fp16), what one ds_read_b64_tr_b16 hands lane L as dim 32md + L%32
 //     of four keys; the keys follow the S^T accumulator's own order, so the
 //     P^T operand is a slice of the accumulator.
-#include "prefill_common.h"
+#include "prefill_merge.h"
 
+#include <climits>
 #include <type_traits>
 
 namespace dd_prefill {
@@ -174,7 +175,11 @@ constexpr int pipe_ring() { return D == 160 ? DD_PF_RING160 : DD_PF_RING; }
 // D is the LDS layout's head size (64, 128, 160 or 256); DR <= D the real one (a
 // multiple of 16 above D / 2): rows are DR elements long in memory, the
 // layout's dims DR .. D-1 are loaded as zeros and skipped by the MFMAs.
-template <int DT, int D, int DR>
+// PLAN: the items come from a plan; otherwise they are numbered, and their keys
+// may be split over workgroups.  (Kernels of their own: the numbering and the
+// split cost scalar registers, 2 % of the planned kernel's time on 8 x 512
+// tokens.)
+template <int DT, int D, int DR, bool PLAN>
 __global__ __launch_bounds__(64 * pipe_waves<D>()) __attribute__((amdgpu_waves_per_eu(pipe_waves<D>() / 4)))
 void prefill_pipe_kernel(PrefillParams p) {
   static_assert(D == 64 || D == 128 || D == 160 || D == 256, "layouts for head sizes 64, 128, 160 and 256");
@@ -216,20 +221,26 @@ void prefill_pipe_kernel(PrefillParams p) {
   char *const s_v = s_kv + NKS * PLANE;
   __shared__ int s_tab[kTabP];
 
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int w = uniform(tid >> 6);
-  const int l32 = lane & 31;
-  const int h2 = lane >> 5;
-
   __shared__ int s_flag;   // some column of this item needs the exact re-run
   // A workgroup runs the plan's items for it one after another (one
   // workgroup per CU: no dispatch gap between them, and the next item's
   // plan entry is known before the current one ends).
-  const int rounds = prefill_rounds(p);
+  const int rounds = PLAN ? prefill_rounds(p) : 1;
   for (int round = 0; round < rounds; ++round) {
+  // In the large layouts opaque to the compiler, so that it does not compute
+  // every address and mask of the prologue and epilogue before the rounds and
+  // keep them in registers through the steady state (the 160 layout spilled 42
+  // VGPRs, now none: 275 -> 263 us on 8 x 512 tokens, the 256 layout 525 ->
+  // 515 us; at 64 and 128 dims, which have the registers, recomputing them in
+  // every round costs 1 %).
+  int tid = threadIdx.x;
+  if constexpr (PLAN && D > 128) asm volatile("" : "+v"(tid));
+  const int lane = tid & 63;
+  const int w = uniform(tid >> 6);
+  const int l32 = lane & 31;
+  const int h2 = lane >> 5;
   PrefillItem it;
-  if (!prefill_item(p, it, round)) break;
+  if (!prefill_item<PLAN>(p, it, round)) break;
   if (round > 0) {
     // every wave has read its previous output tile out of the V ring
     lgkm_drain();
@@ -248,10 +259,9 @@ void prefill_pipe_kernel(PrefillParams p) {
   const long slot = it.slot;
   const int rows_here = min(rows, len - r0);
 
-  const int k_hi = start + r0 + rows_here;  // exclusive
-  const int k_lo = p.window > 0 ? max(0, start + r0 - p.window + 1) : 0;
-  const int kt_first = k_lo / KT;
-  const int kt_last = (k_hi - 1) / KT;
+  int kt_first, kt_last;
+  const int nsplit = prefill_tiles<!PLAN>(p, it, KT, r0, rows_here, kt_first, kt_last);
+  if (!PLAN && it.split >= nsplit) continue;
 
   // page-table entries of the 16-key chunks this item visits
   const int e_first = (kt_first * KT) >> p.page_shift;
@@ -281,7 +291,10 @@ void prefill_pipe_kernel(PrefillParams p) {
 
   // ---- this lane's query column; Q^T operands (B of S^T) ----
   const int col = w * 32 + l32;
-  const int qr = col / G;
+  // c / G of a column c < 256 without a division (exact: c < 65536 / G)
+  const int g_inv = (65536 + G - 1) / G;
+  auto col_row = [&](int c) __attribute__((always_inline)) { return (c * g_inv) >> 16; };
+  const int qr = col_row(col);
   const int gh = col - qr * G;
   const bool colok = qr < rows_here;
   const int qpos = start + r0 + (colok ? qr : 0);
@@ -655,6 +668,32 @@ void prefill_pipe_kernel(PrefillParams p) {
 
   // ---- normalise and store: lane holds dims 32md + 8(r/4) + 4h2 + r%4 of its column ----
   const float l = xor32_sum(l_part);
+  if (!PLAN && nsplit > 1) {
+    // One split of the item: O^T, the offset and the denominator as they are,
+    // every store 1 KiB of consecutive bytes.  prefill_merge_kernel, which
+    // runs next, raises the flag that is cleared here.
+    if constexpr (DT == DD_BF16) {
+      if (p.flags && it.split == 0) {
+        if (tid == 0) p.flags[(long)grp * p.max_tiles + qt] = 0;
+        if (qt == 0)
+          for (int t = (len + rows - 1) / rows + tid; t < p.max_tiles; t += NT) p.flags[(long)grp * p.max_tiles + t] = 0;
+      }
+    }
+    const long unit = ((long)grp * p.max_tiles + qt) * p.max_splits + it.split;
+    float *part = p.part + unit * prefill_part_floats(COLS, DR) + (long)w * prefill_part_floats(32, DR);
+#pragma unroll
+    for (int md = 0; md < MDR; ++md)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4)
+        ((f32x4 *)part)[(md * 4 + q4) * 64 + lane] =
+            f32x4{o[md][4 * q4], o[md][4 * q4 + 1], o[md][4 * q4 + 2], o[md][4 * q4 + 3]};
+    part += 1024 * MDR;
+    if (h2 == 0) {
+      part[l32] = m_run * sc;
+      part[32 + l32] = l;
+    }
+    continue;
+  }
   if constexpr (DT == DD_BF16) {
     if (p.flags) {
       // largest |O| of the column (as bits: infinities and NaNs compare
@@ -711,7 +750,7 @@ void prefill_pipe_kernel(PrefillParams p) {
   for (int e0 = 0; e0 < 32 * PR; e0 += 64) {
     const int e = e0 + lane;
     const int c = e / PR, k = e - (e / PR) * PR;
-    const int cq = (w * 32 + c) / G;
+    const int cq = col_row(w * 32 + c);
     if (e < 32 * PR && cq < rows_here) {
       const int cg = w * 32 + c - cq * G;
       const u32x4 x = *(const u32x4 *)(otile + c * ORS + 16 * k);
@@ -726,11 +765,22 @@ int launch_pipe(PrefillParams p, int max_len, int plan_len, hipStream_t s) {
   constexpr int COLS = 32 * pipe_waves<D>();
   if (COLS / p.G < 1) return DD_EUNSUPPORTED;
   p.max_tiles = (int)dd_cdiv(max_len, COLS / p.G);
-  const long grid = p.plan ? (long)plan_len : 8L * dd_cdiv((long)p.n * p.KH, 8) * p.max_tiles;
+  const long items = (long)p.n * p.KH * p.max_tiles;
+  if (p.plan || p.max_splits <= 1) p.max_splits = 1, p.split_tiles = INT_MAX;
+  const long grid = p.plan ? (long)plan_len : 8L * dd_cdiv(items * p.max_splits, 8);
   if (grid == 0) return DD_OK;
   if (grid > 0x7fffffffL) return DD_EUNSUPPORTED;
-  hipLaunchKernelGGL((prefill_pipe_kernel<DT, D, DR>), dim3((unsigned)grid), dim3(64 * pipe_waves<D>()), 0, s, p);
+  if (p.plan)
+    hipLaunchKernelGGL((prefill_pipe_kernel<DT, D, DR, true>), dim3((unsigned)grid), dim3(64 * pipe_waves<D>()), 0, s, p);
+  else
+    hipLaunchKernelGGL((prefill_pipe_kernel<DT, D, DR, false>), dim3((unsigned)grid), dim3(64 * pipe_waves<D>()), 0, s,
+                       p);
   DD_LAUNCH_CHECK();
+  if (p.max_splits > 1) {
+    hipLaunchKernelGGL((prefill_merge_kernel<DT, pipe_waves<D>(), pipe_keys<D>(), DR>),
+                       dim3((unsigned)items, pipe_waves<D>()), dim3(64 * ((DR + 31) / 32)), 0, s, p);
+    DD_LAUNCH_CHECK();
+  }
   return DD_OK;
 }
 

@@ -77,6 +77,20 @@ def prefill_plan(lengths, starts, heads, kv_heads, dim, window=0, slots=None, wo
 PLAN_INTS = 8   # DD_PREFILL_PLAN_INTS
 
 
+def prefill_split(lengths, starts, heads, kv_heads, dim, dtype, window, device):
+    """(split_tiles, max_splits, scratch floats) of a prefill call on ``device``
+    (dd_prefill_split), or None: a 16-bit call with more work items than CUs,
+    or no kernel that splits."""
+    lengths = np.ascontiguousarray(lengths, dtype=np.int64)
+    starts = np.ascontiguousarray(starts, dtype=np.int64)
+    tiles, splits, floats = ctypes.c_int(0), ctypes.c_int(1), ctypes.c_int64(0)
+    code = _native.library().dd_prefill_split(
+        lengths.ctypes.data_as(ctypes.c_void_p), starts.ctypes.data_as(ctypes.c_void_p), len(lengths), heads, kv_heads,
+        dim, DTYPE_CODES[dtype], int(window or 0), _cu_count(device), ctypes.byref(tiles), ctypes.byref(splits),
+        ctypes.byref(floats))
+    return None if code else (tiles.value, splits.value, floats.value)
+
+
 def prefill_attention(query, cache_k, cache_v, packed, page_table, window=0, scale=None, out=None,
                       segments=None, flags=None):
     """Causal attention of every packed query token over its slot's pages.
@@ -113,10 +127,19 @@ def prepare_prefill(query, cache_k, cache_v, packed, page_table, window=0, scale
         return PrefillLaunch(out, None)
     max_len = max(packed.lengths[a:b])
     max_context = max(s + n for s, n in zip(packed.starts[a:b], packed.lengths[a:b]))
-    plan_dev, plan_len = None, 0
-    if q.dtype != torch.float32 and scale != 0.0 and _has_mfma_geometry(D, H // cache_k.shape[1]):
-        # the MFMA kernel's XCD-balanced workgroup order (the fp32 / other-D
-        # kernel takes none)
+    plan_dev, plan_len, scratch = None, 0, None
+    split = None
+    mfma = q.dtype != torch.float32 and scale != 0.0 and _has_mfma_geometry(D, H // cache_k.shape[1])
+    if mfma:
+        _native.refuse_capture()
+        split = prefill_split(packed.lengths[a:b], packed.starts[a:b], H, cache_k.shape[1], D, q.dtype, window,
+                              q.device)
+    split_tiles, max_splits, floats = split or (0, 1, 0)
+    if floats:
+        scratch = torch.empty(floats, dtype=torch.float32, device=q.device)
+    if mfma and split is None:
+        # more work items than CUs: the MFMA kernel's XCD-balanced workgroup
+        # order (with fewer there is nothing to order, and nothing to upload)
         plan = prefill_plan(packed.lengths[a:b], packed.starts[a:b], H, cache_k.shape[1], D, window,
                             packed.slots[a:b], _persistent_workgroups(q.device, D))
         if len(plan) == 0:
@@ -134,8 +157,9 @@ def prepare_prefill(query, cache_k, cache_v, packed, page_table, window=0, scale
             ptr(packed.cu_seqlens[a:]), ptr(packed.context_lens[a:]), ptr(packed._meta[2, a:]), b - a, max_len,
             max_context, ptr(page_table), page_table.shape[0], page_table.shape[1], H, cache_k.shape[1], D,
             cache_k.shape[2], cache_k.shape[0], int(window or 0), scale,
-            ptr(plan_dev) if plan_dev is not None else None, plan_len, ptr(flags), ptr(out))
-    return PrefillLaunch(out, args, keep=(q, cache_k, cache_v, packed, page_table, plan_dev, flags))
+            ptr(plan_dev), plan_len, ptr(flags), ptr(out), split_tiles, max_splits, ptr(scratch),
+            0 if scratch is None else scratch.numel())
+    return PrefillLaunch(out, args, keep=(q, cache_k, cache_v, packed, page_table, plan_dev, flags, scratch))
 
 
 class PrefillLaunch:
@@ -147,16 +171,13 @@ class PrefillLaunch:
         self.out, self._args, self._keep = out, args, keep
 
     def run(self):
-        if self._args is not None:
-            call('dd_prefill_attention', *self._args,
-                 ctypes.c_void_p(torch.cuda.current_stream(self.out.device).cuda_stream))
-        return self.out
+        return self.phase(3)
 
     def phase(self, which):
         """Enqueue one launch of the call: 1 the attention kernel, 2 the exact
         re-run of the items the bf16 kernel flagged (both together = run())."""
         if self._args is not None:
-            call('dd_prefill_attention_phase', *self._args, int(which),
+            call('dd_prefill_attention_split', *self._args, int(which),
                  ctypes.c_void_p(torch.cuda.current_stream(self.out.device).cuda_stream))
         return self.out
 
@@ -172,6 +193,10 @@ def _persistent_workgroups(device, dim):
     forced = os.environ.get('DAMENDAEMON_AMD_PREFILL_WORKGROUPS')   # tuning: 0 = one item per workgroup
     if forced is not None:
         return int(forced)
+    return _cu_count(device)
+
+
+def _cu_count(device):
     index = torch.device(device).index
     index = torch.cuda.current_device() if index is None else index
     if index not in _CU_COUNT:

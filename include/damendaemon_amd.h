@@ -308,6 +308,42 @@ int dd_prefill_attention_phase(const void *q, const void *k, const void *v,
                                int phase, void *stream);
 
 /*
+ * dd_prefill_attention_phase (phase as there) with the keys of every work
+ * item split into shares of split_tiles key tiles, run by workgroups of
+ * their own and combined by a third launch (part of phase 1): for calls with
+ * too few work items to fill the GPU.  plan must be NULL when max_splits > 1.
+ *   max_splits   splits of the longest item; 1: not split (split_tiles and
+ *                scratch unused), the schedule as in dd_prefill_attention
+ *   scratch      device fp32 workspace of at least the scratch_floats that
+ *                dd_prefill_split returns (else DD_ESCRATCH); needs no
+ *                clearing, written and read by this call only
+ * No reference counterpart.
+ */
+int dd_prefill_attention_split(const void *q, const void *k, const void *v,
+                               int dtype, const int64_t *cu_seqlens,
+                               const int64_t *context_lens, const int64_t *slots,
+                               int n, int max_len, int max_context,
+                               const int32_t *page_table, int table_rows,
+                               int table_width, int heads, int kv_heads,
+                               int dim, int page_size, int64_t capacity,
+                               int window, float scale, const int32_t *plan,
+                               int plan_len, int32_t *flags, void *out,
+                               int split_tiles, int max_splits, float *scratch,
+                               int64_t scratch_floats, int phase, void *stream);
+
+/*
+ * How dd_prefill_attention_split should run these segments (HOST int64
+ * arrays, as in dd_prefill_plan) on `workgroups` CUs.  DD_EUNSUPPORTED: a
+ * 16-bit call with more work items than CUs (dd_prefill_plan's schedule
+ * balances them), or no kernel that splits; DD_OK: no plan is needed, and the three
+ * outputs are dd_prefill_attention_split's arguments.
+ */
+int dd_prefill_split(const int64_t *lengths, const int64_t *starts, int n,
+                     int heads, int kv_heads, int dim, int dtype, int window,
+                     int workgroups, int *split_tiles, int *max_splits,
+                     int64_t *scratch_floats);
+
+/*
  * Entries of dd_prefill_attention's flags workspace for these arguments (0
  * when the call needs none); negative = -DD_E*.  No reference counterpart:
  * the exactness guard of the fp16 P.V product of bf16 pages.

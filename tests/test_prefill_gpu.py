@@ -413,3 +413,51 @@ def test_prefill_phases_equal_one_call():
     launch.phase(2)
     assert torch.equal(launch.out, whole)
     assert torch.isfinite(whole.float()).all()
+
+
+# Few work items on long histories: the keys are split over workgroups (dd_prefill_split).
+@pytest.mark.parametrize('dim,heads,kvh', [(128, 14, 2), (64, 8, 1), (48, 4, 4), (96, 8, 2), (160, 4, 1), (176, 4, 2),
+                                           (256, 16, 2)])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('window', [0, 1400])
+def test_prefill_split_keys(dim, heads, kvh, dtype, window):
+    """Segments with many shares, few and one, a last share of one key, a row that sees
+    none of a share, windows that drop the first shares; and a launch of two phases."""
+    lengths, starts = [70, 1, 33, 5], [3000, 2048, 0, 767]
+    case, q, slots = build(lengths, starts, heads, kvh, dim, dtype, seed=dim + heads + window)
+    table = case['page_table'].to(DEV)
+    split = ragged.prefill_split(lengths, starts, heads, kvh, dim, dtype, window, DEV)
+    assert split is not None and split[1] > 1, split
+    packed = packing.pack_batch(lengths, starts, slots, table)
+    launch = ragged.prepare_prefill(q.to(DEV), case['cache_k'].to(DEV), case['cache_v'].to(DEV), packed, table,
+                                    window=window)
+    out = launch.run().clone()
+    exp = O.prefill_attention(q, case['cache_k'], case['cache_v'], lengths, starts, slots, case['page_table'],
+                              window=window)
+    check(out, exp)
+    launch.out.fill_(float('nan'))
+    launch.phase(1)
+    launch.phase(2)
+    assert torch.equal(launch.out, out)
+
+
+def test_prefill_split_keys_rerun():
+    """V past fp16's range in one share of one KV head: that head's items are flagged by the
+    merge and recomputed, the others' flags are cleared, with NaN in unused pages."""
+    lengths, starts = [130, 9], [2900, 1500]
+    heads, kvh, dim = 8, 2, 128
+    case, q, slots = build(lengths, starts, heads, kvh, dim, torch.bfloat16, seed=19)
+    case['cache_v'][int(case['page_table'][0, 100]), 1, 3] = 3e5
+    table = case['page_table'].to(DEV)
+    packed = packing.pack_batch(lengths, starts, slots, table)
+    assert ragged.prefill_split(lengths, starts, heads, kvh, dim, torch.bfloat16, 0, DEV)[1] > 1
+    rows = 256 // (heads // kvh)
+    tiles = -(-130 // rows)
+    flags = torch.full((2 * kvh * tiles,), 7, dtype=torch.int32, device=DEV)
+    out = ragged.prefill_attention(q.to(DEV), case['cache_k'].to(DEV), case['cache_v'].to(DEV), packed, table,
+                                   flags=flags)
+    hot = {(0 * kvh + 1) * tiles + t for t in range(-(-130 // rows))}
+    assert flags.cpu().tolist() == [int(i in hot) for i in range(2 * kvh * tiles)]
+    exp = O.prefill_attention(q, case['cache_k'], case['cache_v'], lengths, starts, slots, case['page_table'])
+    exp_abs = O.prefill_attention(q, case['cache_k'], case['cache_v'].abs(), lengths, starts, slots, case['page_table'])
+    assert _relative_error(out, exp, exp_abs) <= 2e-3

@@ -140,3 +140,31 @@ def test_persistent_plan_rounds(seed):
     for x in range(8):
         ls = load[x::8]
         assert max(ls) - min(ls) <= biggest + 2 * rounds + 2   # the schedule also charges 2 per item
+
+
+@pytest.mark.parametrize('seed', range(40))
+def test_split_shares(seed):
+    """dd_prefill_split: None exactly when there are more items than workgroups; else shares of
+    at least four tiles that keep the units at one per workgroup, and the scratch they need."""
+    rng = random.Random(seed)
+    dim = rng.choice(DIMS)
+    kv_heads = rng.choice([1, 2, 8])
+    heads = kv_heads * rng.choice([1, 4, 7])
+    lengths = [rng.choice([1, 7, 64, 300, 512, 2000]) for _ in range(rng.randint(1, 6))]
+    starts = [rng.choice([0, rng.randint(0, 300), rng.randint(0, 30000)]) for _ in lengths]
+    window, workgroups = rng.choice([0, 0, 700]), rng.choice([64, 256])
+    cost, max_tiles = _items(lengths, starts, heads, kv_heads, dim, window)
+    tiles, splits, floats = ctypes.c_int(), ctypes.c_int(), ctypes.c_int64()
+    arrays = [np.array(x, dtype=np.int64) for x in (lengths, starts)]
+    code = _native.library().dd_prefill_split(*(a.ctypes.data_as(ctypes.c_void_p) for a in arrays), len(lengths), heads,
+                                              kv_heads, dim, _native.BF16, window, workgroups, ctypes.byref(tiles),
+                                              ctypes.byref(splits), ctypes.byref(floats))
+    assert (code == 0) == (len(cost) <= workgroups)
+    if code or splits.value == 1:
+        assert splits.value == 1 and floats.value == 0
+        return
+    longest = max(cost.values())
+    assert 4 <= tiles.value <= longest - 4 and splits.value == -(-longest // tiles.value)
+    assert sum(-(-c // tiles.value) for c in cost.values()) <= workgroups
+    per = ROWS[dim] // 32 * (32 * (-(-dim // 32) * 32) + 64)     # per unit: O^T, offsets and denominators
+    assert floats.value == len(lengths) * kv_heads * max_tiles * splits.value * per <= 1 << 28
