@@ -52,6 +52,10 @@ static bool geometry(int D, Geometry *g) {
   return true;
 }
 
+// prefill_x3_kernel: fp32 pages
+constexpr int kX3Cols = 256;
+static bool x3_dim(int D) { return D > 0 && D <= 128 && D % 16 == 0; }
+
 template <int DT>
 int dispatch(const PrefillParams &p, int D, int max_len, int plan_len, hipStream_t s) {
   return pipe_dim(D) ? prefill_pipe_dispatch(p, DT, D, max_len, plan_len, s) : DD_EUNSUPPORTED;
@@ -134,6 +138,30 @@ static int prefill_entry(int phase, const void *q, const void *k, const void *v,
     const int rc = dd_prefill_f32(args, dtype, s);
     return rc != DD_EUNSUPPORTED ? rc : dd_prefill_generic(args, dtype, s);
   };
+  // fp32 pages with a workspace: split products on the bf16 matrix cores, and
+  // the items whose result is not finite again on the fp32 ones
+  if (dtype == DD_F32 && part && x3_dim(dim) && p.G <= kX3Cols) {
+    const long items = (long)n * kv_heads * dd_cdiv(max_len, kX3Cols / p.G);
+    if (max_splits > 1 && (split_tiles < 1 || plan)) return DD_EINVAL;
+    const long flag_floats = dd_cdiv(items, 64) * 64;
+    if (part_floats < flag_floats ||
+        (max_splits > 1 && (part_floats - flag_floats) / prefill_part_floats(kX3Cols, dim) / max_splits < items))
+      return DD_ESCRATCH;
+    p.flags = (int32_t *)part;
+    p.part = part + flag_floats;
+    p.split_tiles = split_tiles;
+    p.max_splits = max_splits;
+    p.scale_log2 = a.scale_log2;
+    if (phase & 1) {
+      const int rc = prefill_x3_dispatch(p, dim, max_len, s);
+      if (rc != DD_OK) return rc;
+    }
+    if (!(phase & 2)) return DD_OK;
+    a.flags = p.flags;
+    a.flag_rows = kX3Cols / p.G;
+    a.flag_tiles = (int)dd_cdiv(max_len, a.flag_rows);
+    return exact(a);
+  }
   // (and more query heads per KV head than one 16-bit work item has columns)
   if (dtype == DD_F32 || !geometry(dim, &geom) || geom.cols < heads / kv_heads || scale == 0.f)
     return (phase & 1) ? exact(a) : DD_OK;
@@ -219,8 +247,10 @@ extern "C" int dd_prefill_split(const int64_t *lengths, const int64_t *starts, i
   *split_tiles = 0;
   *max_splits = 1;
   *scratch_floats = 0;
-  Geometry g;
-  if (dtype == DD_F32 || !geometry(dim, &g) || g.cols < heads / kv_heads) return DD_EUNSUPPORTED;
+  const bool x3 = dtype == DD_F32;
+  Geometry g{kX3Cols, DD_PREFILL_X3_KEYS};
+  if (x3 ? !x3_dim(dim) : !geometry(dim, &g)) return DD_EUNSUPPORTED;
+  if (g.cols < heads / kv_heads) return DD_EUNSUPPORTED;
   const int rows = g.cols / (heads / kv_heads);
   long items = 0, max_tiles = 0;
   for (int i = 0; i < n; ++i) {
@@ -231,7 +261,9 @@ extern "C" int dd_prefill_split(const int64_t *lengths, const int64_t *starts, i
   items *= kv_heads;
   const long grid_items = (long)n * kv_heads * max_tiles;
   if (grid_items > 0x7fffffffL) return DD_EUNSUPPORTED;
-  if (items > workgroups) return DD_EUNSUPPORTED;   // enough items: dd_prefill_plan's schedule
+  const long flag_floats = x3 ? dd_cdiv(grid_items, 64) * 64 : 0;
+  *scratch_floats = flag_floats;
+  if (!x3 && items > workgroups) return DD_EUNSUPPORTED;   // enough items: dd_prefill_plan's schedule
   // units of the call with shares of `share` tiles; the longest item's tiles and all items'
   long longest = 0, total = 0;
   auto units = [&](long share) {
@@ -255,21 +287,43 @@ extern "C" int dd_prefill_split(const int64_t *lengths, const int64_t *starts, i
   // the grid and the scratch are those of the longest item for all: at most 1 GiB
   const long most = per > 0 ? std::max(1L, (1L << 28) / per) : 1;
   long share = longest;
-  long lo = kLeast, hi = longest;   // (one share per item always fits)
-  while (lo < hi) {
-    const long mid = (lo + hi) / 2;
-    if (units(mid) <= workgroups) hi = mid; else lo = mid + 1;
-  }
-  if (longest - lo >= kGain) {
-    // (equal shares of the longest item where they keep to the units above)
-    const long splits = std::min(dd_cdiv(longest, lo), most);
-    const long even = std::max(kLeast, dd_cdiv(longest, splits));
-    share = units(even) <= workgroups ? even : lo;
+  if (x3) {
+    // Also with more units than CUs, where a whole item is a large part of the
+    // call and leaves CUs idle at its end: the share with the least estimated
+    // time.  One at a time on every CU while they last, else the average load
+    // and half a unit; a unit's start and end are about four tiles' time, the
+    // merge about three.
+    auto estimate = [&](long s, long splits) {
+      const double u = (double)units(s), unit = (double)s + 4;
+      const double load = u <= workgroups ? unit : (total + 4 * u) / workgroups + unit / 2;
+      return load + (splits > 1 ? 3 : 0);
+    };
+    double best = estimate(longest, 1) * 0.95;
+    for (long k = 2; k <= std::min(most, 32L) && longest >= kLeast * k; ++k) {
+      const long s = dd_cdiv(longest, k);
+      const double e = estimate(s, k);
+      if (e < best) {
+        best = e;
+        share = s;
+      }
+    }
+  } else {
+    long lo = kLeast, hi = longest;   // (one share per item always fits)
+    while (lo < hi) {
+      const long mid = (lo + hi) / 2;
+      if (units(mid) <= workgroups) hi = mid; else lo = mid + 1;
+    }
+    if (longest - lo >= kGain) {
+      // (equal shares of the longest item where they keep to the units above)
+      const long splits = std::min(dd_cdiv(longest, lo), most);
+      const long even = std::max(kLeast, dd_cdiv(longest, splits));
+      share = units(even) <= workgroups ? even : lo;
+    }
   }
   if (share >= longest) return DD_OK;
   *split_tiles = (int)share;
   *max_splits = (int)dd_cdiv(longest, share);
-  *scratch_floats = per * *max_splits;
+  *scratch_floats = flag_floats + per * *max_splits;
   return DD_OK;
 }
 

@@ -63,11 +63,13 @@ DD_DEV void prefill_segment(const PrefillParams &p, PrefillItem &it) {
 // stores the count (field 5).
 DD_DEV int prefill_rounds(const PrefillParams &p) { return p.plan[(long)kPlanInts * blockIdx.x + 5]; }
 // Item of round `round` of this workgroup; false: nothing to do.  Without a
-// plan the units (group, split, query tile), query tiles innermost and
-// longest first, are cut into 8 runs of equal length, one per XCD
-// (consecutive workgroups go to the 8 XCDs round-robin, each with its own
-// L2), so that the query tiles that read the same keys share an L2 and no XCD
-// gets more workgroups than another.
+// plan workgroup b is unit (split, query tile, group), groups innermost:
+// consecutive workgroups go to the 8 XCDs round-robin, each with its own L2,
+// so with KV heads in multiples of 8 all units that read one KV head's keys
+// share an L2, and every XCD gets the same share of the long segments, of the
+// late query tiles and of the first (full) splits, which start first.  (Runs
+// of consecutive units per XCD kept the L2 as well, but gave an XCD one
+// segment's heads: 8 ragged fp32 segments left CUs idle 36 % of the time.)
 template <bool PLAN>
 DD_DEV bool prefill_item(const PrefillParams &p, PrefillItem &it, int round) {
   if constexpr (PLAN) {
@@ -84,15 +86,11 @@ DD_DEV bool prefill_item(const PrefillParams &p, PrefillItem &it, int round) {
     it.split = 0;
     return it.grp < p.n * p.KH;
   } else {
-    const int units = p.n * p.KH * p.max_splits * p.max_tiles;
-    const int per_xcd = (units + 7) / 8;
-    const int j = blockIdx.x >> 3;
-    const int u = (int)(blockIdx.x & 7) * per_xcd + j;
-    if (j >= per_xcd || u >= units) return false;
-    const int gs = u / p.max_tiles;
-    it.grp = gs / p.max_splits;
-    it.split = gs - it.grp * p.max_splits;
-    it.qt = p.max_tiles - 1 - (u - gs * p.max_tiles);
+    const int ngrp = p.n * p.KH;
+    const int r = blockIdx.x / ngrp;
+    it.grp = blockIdx.x - r * ngrp;
+    it.split = r / p.max_tiles;
+    it.qt = p.max_tiles - 1 - (r - it.split * p.max_tiles);
     prefill_segment(p, it);
     return true;
   }
@@ -141,6 +139,13 @@ constexpr int kBufferWord3 = 0x00020000;
 
 typedef __attribute__((address_space(3))) void lds_void;
 
+// Keys per tile of prefill_x3_kernel (its columns per work item: 256).
+#define DD_PREFILL_X3_KEYS 32
+// Below this a whole result row may miss the parts of V under 2^-126 that its
+// bf16 products lose (2^-26 of it).
+constexpr float kX3Least = 0x1p-100f;
+
 int prefill_pipe_dispatch(const PrefillParams &p, int dtype, int dim, int max_len, int plan_len, hipStream_t s);
+int prefill_x3_dispatch(const PrefillParams &p, int dim, int max_len, hipStream_t s);
 
 }  // namespace dd_prefill

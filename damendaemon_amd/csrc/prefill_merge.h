@@ -1,4 +1,4 @@
-// The combine of split prefill work items (prefill_pipe.hip).
+// The combine of split prefill work items (prefill_pipe.hip, prefill_x3.hip).
 #pragma once
 
 #include "prefill_common.h"
@@ -12,7 +12,8 @@ namespace {
 // load is 1 KiB of consecutive bytes.  Reads kBatch splits at a time (all
 // loads in flight), as the decode merge does.  Items whose result has to be
 // recomputed exactly raise their flag: bf16 ones that show V outside fp16's
-// normal range (see prefill_pipe_kernel).  NW, KT: waves and keys per tile of the split kernel.
+// normal range (see prefill_pipe_kernel), fp32 ones that are not finite or tiny
+// (see prefill_x3_kernel).  NW, KT: waves and keys per tile of the split kernel.
 template <int DT, int NW, int KT, int DR>
 __global__ __launch_bounds__(64 * ((DR + 31) / 32)) void prefill_merge_kernel(PrefillParams p) {
   constexpr int MDR = (DR + 31) / 32;
@@ -78,7 +79,7 @@ __global__ __launch_bounds__(64 * ((DR + 31) / 32)) void prefill_merge_kernel(Pr
     }
     m = top;
   }
-  if constexpr (DT == DD_BF16) {
+  if constexpr (DT != DD_F16) {
     if (p.flags) {
       unsigned mb = 0;
 #pragma unroll
@@ -92,7 +93,7 @@ __global__ __launch_bounds__(64 * ((DR + 31) / 32)) void prefill_merge_kernel(Pr
 #pragma unroll
         for (int k = 1; k < MDR; ++k) mb = max(mb, s_top[k][l32]);
         const float top = __uint_as_float(mb) / l;
-        const bool fine = top >= 0x1p-12f && top <= 3.0e38f;
+        const bool fine = top >= (DT == DD_F32 ? kX3Least : 0x1p-12f) && top <= 3.0e38f;
         if (__builtin_amdgcn_ballot_w64(colok && !fine) && lane == 0)
           p.flags[blockIdx.x] = 1;
       }
@@ -105,8 +106,11 @@ __global__ __launch_bounds__(64 * ((DR + 31) / 32)) void prefill_merge_kernel(Pr
   for (int q = 0; q < 4; ++q) {
     const int d = 32 * md + 8 * q + 4 * h2;
     if (DR % 32 && d >= DR) continue;
-    *(u32x2 *)((unsigned short *)p.out + row + d) =
-        u32x2{pack2<DT>(o[q][0] * inv, o[q][1] * inv), pack2<DT>(o[q][2] * inv, o[q][3] * inv)};
+    if constexpr (DT == DD_F32)
+      *(f32x4 *)((float *)p.out + row + d) = o[q] * inv;
+    else
+      *(u32x2 *)((unsigned short *)p.out + row + d) =
+          u32x2{pack2<DT>(o[q][0] * inv, o[q][1] * inv), pack2<DT>(o[q][2] * inv, o[q][3] * inv)};
   }
 }
 

@@ -767,7 +767,7 @@ int launch_pipe(PrefillParams p, int max_len, int plan_len, hipStream_t s) {
   p.max_tiles = (int)dd_cdiv(max_len, COLS / p.G);
   const long items = (long)p.n * p.KH * p.max_tiles;
   if (p.plan || p.max_splits <= 1) p.max_splits = 1, p.split_tiles = INT_MAX;
-  const long grid = p.plan ? (long)plan_len : 8L * dd_cdiv(items * p.max_splits, 8);
+  const long grid = p.plan ? (long)plan_len : items * p.max_splits;
   if (grid == 0) return DD_OK;
   if (grid > 0x7fffffffL) return DD_EUNSUPPORTED;
   if (p.plan)

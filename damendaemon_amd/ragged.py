@@ -132,6 +132,7 @@ def prepare_prefill(query, cache_k, cache_v, packed, page_table, window=0, scale
     mfma = q.dtype != torch.float32 and scale != 0.0 and _has_mfma_geometry(D, H // cache_k.shape[1])
     if mfma:
         _native.refuse_capture()
+    if mfma or q.dtype == torch.float32:
         split = prefill_split(packed.lengths[a:b], packed.starts[a:b], H, cache_k.shape[1], D, q.dtype, window,
                               q.device)
     split_tiles, max_splits, floats = split or (0, 1, 0)

@@ -316,7 +316,11 @@ int dd_prefill_attention_phase(const void *q, const void *k, const void *v,
  *                scratch unused), the schedule as in dd_prefill_attention
  *   scratch      device fp32 workspace of at least the scratch_floats that
  *                dd_prefill_split returns (else DD_ESCRATCH); needs no
- *                clearing, written and read by this call only
+ *                clearing, written and read by this call only.  fp32 pages
+ *                at head sizes that are multiples of 16 up to 128 need it
+ *                unsplit too: with one they run on the bf16 matrix cores
+ *                (products of three-part splits, fp32 accurate), without
+ *                (NULL) on the fp32 ones
  * No reference counterpart.
  */
 int dd_prefill_attention_split(const void *q, const void *k, const void *v,

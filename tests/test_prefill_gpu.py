@@ -461,3 +461,73 @@ def test_prefill_split_keys_rerun():
     exp = O.prefill_attention(q, case['cache_k'], case['cache_v'], lengths, starts, slots, case['page_table'])
     exp_abs = O.prefill_attention(q, case['cache_k'], case['cache_v'].abs(), lengths, starts, slots, case['page_table'])
     assert _relative_error(out, exp, exp_abs) <= 2e-3
+
+
+# Of a row's sum p|v|: a logit is rounded to 2^-24 of sums of size |q||k| / sqrt(dim), 16 or less here, which
+# moves its probability by as much, and the sums of products and of probabilities add a few roundings.
+FP32_BOUND = 32 * 2.0 ** -24
+
+
+def _fp32_error(out, exp, exp_abs):
+    a = out.cpu().double()
+    assert torch.isfinite(a).all(), 'non-finite output'
+    err = ((a - exp).abs() / exp_abs.amax(dim=-1, keepdim=True)).max().item()
+    print(f'error {err:.3e} of the row magnitude')
+    return err
+
+
+@pytest.mark.parametrize('dim,heads,kvh', [(16, 4, 4), (32, 14, 2), (48, 8, 8), (80, 9, 3), (112, 4, 2), (128, 28, 4)])
+@pytest.mark.parametrize('window', [0, 500])
+def test_prefill_fp32_split_products(dim, heads, kvh, window):
+    """fp32 pages on the bf16 matrix cores (three-part products): split and whole items, one-row and
+    one-key segments, and an error against 64 bits of a few fp32 roundings of the row's magnitude."""
+    lengths, starts = [1, 90, 7, 64], [0, 1500, 2300, 0]
+    case, q, slots = build(lengths, starts, heads, kvh, dim, torch.float32, seed=dim + window)
+    table = case['page_table'].to(DEV)
+    packed = packing.pack_batch(lengths, starts, slots, table)
+    assert ragged.prefill_split(lengths, starts, heads, kvh, dim, torch.float32, window, DEV)[1] > 1
+    for a, b in ((0, 4), (0, 1), (3, 4)):       # split; one key; 64 keys, whole
+        got = ragged.prefill_attention(q.to(DEV), case['cache_k'].to(DEV), case['cache_v'].to(DEV), packed, table,
+                                       window=window, segments=(a, b)).cpu()
+        exp, exp_abs = (O.prefill_attention(q, case['cache_k'], v, lengths, starts, slots, case['page_table'],
+                                            window=window) for v in (case['cache_v'], case['cache_v'].abs()))
+        rows = slice(sum(lengths[:a]), sum(lengths[:b]))
+        assert _fp32_error(got[rows], exp[rows], exp_abs[rows]) <= FP32_BOUND
+
+
+@pytest.mark.parametrize('scale_v', [1e-36, 1e30, 1e35])
+def test_prefill_fp32_split_products_range(scale_v):
+    """V down to where its low parts are subnormal and up to where sums near fp32's limit."""
+    lengths, starts = [40], [700]
+    case, q, slots = build(lengths, starts, 8, 2, 64, torch.float32, seed=3)
+    cv = case['cache_v'] * scale_v
+    table = case['page_table'].to(DEV)
+    packed = packing.pack_batch(lengths, starts, slots, table)
+    got = ragged.prefill_attention(q.to(DEV), case['cache_k'].to(DEV), cv.to(DEV), packed, table)
+    exp, exp_abs = (O.prefill_attention(q, case['cache_k'], v, lengths, starts, slots, case['page_table'])
+                    for v in (cv, cv.abs()))
+    assert _fp32_error(got, exp, exp_abs) <= FP32_BOUND
+
+
+def test_prefill_fp32_split_products_non_finite():
+    """Infinite keys and values, and a value that rounds past bf16's largest: those items come out as
+    fp32 arithmetic gives them (a key of -inf logit is not attended), the others are not disturbed."""
+    lengths, starts = [70, 5], [1300, 0]
+    heads, kvh, dim = 6, 3, 64
+    case, q, slots = build(lengths, starts, heads, kvh, dim, torch.float32, seed=8)
+    ck, cv, table = case['cache_k'].clone(), case['cache_v'].clone(), case['page_table']
+    q[:, 0:2, 5] = q[:, 0:2, 5].abs() + .1
+    ck[int(table[0, 20]), 0, 3, 5] = -math.inf      # KV head 0: its logit is -inf for every query row
+    cv[int(table[0, 30]), 1, 2, 7] = math.inf       # KV head 1: channel 7 is infinite
+    ck[int(table[0, 40]), 2, 2, 9] = 3.4e38         # KV head 2: finite in fp32, not as a bf16 part, and
+    q[:70, 4:6, 9] = 0                              # multiplied by 0
+    q[70:] *= 2.0 ** -115                           # segment 1: queries whose low parts are lost,
+    ck[int(table[1, 0])] *= 2.0 ** 115              # keys that make up for it
+    packed = packing.pack_batch(lengths, starts, slots, table.to(DEV))
+    got = ragged.prefill_attention(q.to(DEV), ck.to(DEV), cv.to(DEV), packed, table.to(DEV)).cpu()
+    exp, exp_abs = (O.prefill_attention(q, ck, v, lengths, starts, slots, table) for v in (cv, cv.abs()))
+    assert torch.isposinf(got[:70, 2:4, 7]).all()
+    got[:70, 2:4, 7] = 0
+    exp[:70, 2:4, 7] = exp_abs[:70, 2:4, 7] = 0
+    assert torch.isfinite(got).all()
+    assert _fp32_error(got, exp, exp_abs) <= FP32_BOUND
