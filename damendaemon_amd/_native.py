@@ -39,6 +39,7 @@ SIGNATURES = {
 SIGNATURES['dd_quantize_q8'] = [_p, _i, _i64, _i, _i, _p, _p, _p]
 SIGNATURES['dd_dequantize_q8'] = [_p, _p, _i64, _i, _i, _p, _i, _p]
 SIGNATURES['dd_pack_batch'] = [_p, _p, _p, _i, _i64, _i64, _p, _i, _i, _i] + [_p] * 9
+SIGNATURES['dd_pack_batch_host'] = [_p, _p, _p, _i, _i64, _i64, _p, _i, _i, _i] + [_p] * 10
 SIGNATURES['dd_store_kv_pages'] = [_p, _p, _i, _p, _i64, _i, _i, _i, _i64, _p, _p, _p]
 SIGNATURES['dd_store_kv_pages_q8'] = [_p, _p, _i, _p, _i64, _i, _i, _i, _i, _i64, _p, _p, _p, _p, _p]
 SIGNATURES['dd_copy_pages'] = [_p, _p, _i, _i, _p, _i, _i64, _i64, _i64, _i, _i, _i, _i, _p]
@@ -51,6 +52,7 @@ SIGNATURES['dd_prefill_attention_phase'] = SIGNATURES['dd_prefill_attention'][:-
 SIGNATURES['dd_prefill_attention_split'] = SIGNATURES['dd_prefill_attention'][:-1] + [_i, _i, _p, _i64, _i, _p]
 SIGNATURES['dd_prefill_split'] = [_p, _p, _i, _i, _i, _i, _i, _i, _i, ctypes.POINTER(_i), ctypes.POINTER(_i),
                                   ctypes.POINTER(_i64)]
+SIGNATURES['dd_prefill_prepare'] = [_p, _p, _i, _i, _i, _i, _i, _i, _f, _i, _p]
 SIGNATURES['dd_prefill_plan'] = [_p, _p, _p, _i, _i, _i, _i, _i, _i, _p, _i]
 SIGNATURES['dd_prefill_geometry'] = [_i, ctypes.POINTER(_i), ctypes.POINTER(_i)]
 SIGNATURES['dd_prefill_indices'] = [_i64, _i, _i, _i64, _i64, _p, _p]
@@ -83,24 +85,43 @@ def library():
     return handle
 
 
-def call(name, *args):
-    lib = library()
-    code = getattr(lib, name)(*args)
+UNSUPPORTED = 2   # DD_EUNSUPPORTED
+
+
+def status(name, *args):
+    """The entry point's return code."""
+    return getattr(library(), name)(*args)
+
+
+def check(name, code):
     if code:
-        raise NativeError(f'{name} failed: {lib.dd_error_string(code).decode()} ({code})')
+        raise NativeError(f'{name} failed: {library().dd_error_string(code).decode()} ({code})')
+
+
+def call(name, *args):
+    code = getattr(library(), name)(*args)
+    if code:
+        check(name, code)
 
 
 def ptr(tensor):
-    return None if tensor is None else ctypes.c_void_p(tensor.data_ptr())
+    """Device address for a c_void_p argument (an int: ctypes converts it, and
+    building a c_void_p object for each costs more than the call)."""
+    return None if tensor is None else tensor.data_ptr()
+
+
+def stream_on(index):
+    """hipStream_t of the current stream of device ``index``, as an int."""
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def stream_of(tensor):
-    return ctypes.c_void_p(torch.cuda.current_stream(tensor.device).cuda_stream)
+    return stream_on(tensor.get_device())
 
 
 def require_device(*tensors):
     for t in tensors:
-        if t is not None and t.device.type != 'cuda':
+        if t is not None and not t.is_cuda:
             raise ValueError('damendaemon_amd kernels need tensors on the GPU '
                              '(there is no CPU path)')
 

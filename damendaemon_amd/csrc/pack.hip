@@ -16,6 +16,11 @@
 // Segment-level prefix sums run in one workgroup (wave-level scans through
 // LDS); the per-token and per-page outputs are filled by a grid of
 // workgroups that locate their segment by binary search in the prefix.
+//
+// Segments known on the host (dd_pack_batch_host) travel in the kernel's own
+// arguments, kPackSegs per launch, and one launch fills everything: every
+// workgroup scans the launch's segments in LDS (no segment waits for another
+// launch's scan), so there is no upload and no second launch.
 #include "common.h"
 #include "q8.h"
 
@@ -129,6 +134,79 @@ __global__ __launch_bounds__(256) void fill_pages_kernel(const int32_t *cu_pages
   gather[k] = (slot >= 0 && slot < table_rows && entry < table_w) ? table[slot * table_w + entry] : -1;
 }
 
+// Segments of one dd_pack_batch_host launch: numbers i0 .. i0 + n of the batch,
+// the first of them at token tok0 and gather entry page0.
+constexpr int kPackSegs = 256;
+struct PackSegs {
+  int n, i0, total;      // total: segments of the whole batch (row stride of meta)
+  int tok_blocks;        // workgroups of the tokens; the ones after them fill the page gather
+  long tok0, page0;
+  int len[kPackSegs], start[kPackSegs], slot[kPackSegs];
+};
+struct PackOut {
+  int64_t *cu, *ends, *context, *meta, *positions, *slot_ids, *slot_map;
+  int32_t *cu_pages, *gather;
+};
+
+__global__ __launch_bounds__(kPackSegs) void pack_segments_kernel(PackSegs segs, const int32_t *table, int table_rows,
+                                                                  int table_w, int page, PackOut out) {
+  __shared__ long s_tmp[16];
+  __shared__ int s_cu[kPackSegs + 1], s_cp[kPackSegs + 1], s_start[kPackSegs], s_slot[kPackSegs];
+  const int i = threadIdx.x;
+  const int len = i < segs.n ? segs.len[i] : 0;
+  const int start = i < segs.n ? segs.start[i] : 0;
+  const int slot = i < segs.n ? segs.slot[i] : 0;
+  const long ctx = (long)start + len;
+  const int np = (int)((ctx + page - 1) / page);
+  // both prefix sums in one scan: tokens in the low half, pages in the high one
+  const long both = block_scan((long)len | ((long)np << 32), s_tmp);
+  const int cu = (int)both, cp = (int)(both >> 32);
+  s_cu[i + 1] = cu;
+  s_cp[i + 1] = cp;
+  s_start[i] = start;
+  s_slot[i] = slot;
+  if (i == 0) s_cu[0] = s_cp[0] = 0;
+  __syncthreads();
+  if (blockIdx.x == 0 && i < segs.n) {
+    const int g = segs.i0 + i;
+    out.cu[g + 1] = segs.tok0 + cu;
+    out.ends[g] = segs.tok0 + cu - 1;
+    out.context[g] = ctx;
+    out.meta[g] = len;
+    out.meta[segs.total + g] = start;
+    out.meta[2L * segs.total + g] = slot;
+    if (out.cu_pages) out.cu_pages[g + 1] = (int32_t)(segs.page0 + cp);
+    if (g == 0) {
+      out.cu[0] = 0;
+      if (out.cu_pages) out.cu_pages[0] = 0;
+    }
+  }
+  if ((int)blockIdx.x < segs.tok_blocks) {
+    const int t = blockIdx.x * kPackSegs + i;
+    if (t >= s_cu[segs.n]) return;
+    int k = find_segment(s_cu, segs.n, t);
+    while (k + 1 < segs.n && s_cu[k + 1] <= t) ++k;   // (empty segments)
+    const long pos = (long)s_start[k] + (t - s_cu[k]);
+    const long sl = s_slot[k];
+    out.positions[segs.tok0 + t] = pos;
+    out.slot_ids[segs.tok0 + t] = sl;
+    if (out.slot_map) {
+      const long entry = pos / page;
+      long phys = -1;
+      if (sl >= 0 && sl < table_rows && entry < table_w) phys = table[sl * table_w + entry];
+      out.slot_map[segs.tok0 + t] = phys * page + (pos - entry * page);
+    }
+    return;
+  }
+  const int e = ((int)blockIdx.x - segs.tok_blocks) * kPackSegs + i;
+  if (e >= s_cp[segs.n]) return;
+  int k = find_segment(s_cp, segs.n, e);
+  while (k + 1 < segs.n && s_cp[k + 1] <= e) ++k;
+  const long sl = s_slot[k];
+  const long entry = e - s_cp[k];
+  out.gather[segs.page0 + e] = (sl >= 0 && sl < table_rows && entry < table_w) ? table[sl * table_w + entry] : -1;
+}
+
 // One thread moves 16 bytes of one (token, KV head) row into its page slot.
 __global__ __launch_bounds__(256) void store_pages_kernel(const char *key, const char *value,
                                                           const int64_t *slot_map, long tokens, int kv_heads,
@@ -240,6 +318,54 @@ extern "C" int dd_pack_batch(const int64_t *lengths, const int64_t *starts, cons
     hipLaunchKernelGGL(fill_pages_kernel, dim3((unsigned)dd_cdiv(total_pages, 256)), dim3(256), 0, s, cu_pages,
                        slots, n, (long)total_pages, page_table, table_rows, table_width, gather_pages);
     DD_LAUNCH_CHECK();
+  }
+  return DD_OK;
+}
+
+extern "C" int dd_pack_batch_host(const int64_t *lengths, const int64_t *starts, const int64_t *slots, int n,
+                                  int64_t total_tokens, int64_t total_pages, const int32_t *page_table,
+                                  int table_rows, int table_width, int page_size, int64_t *cu_seqlens, int64_t *ends,
+                                  int64_t *context_lens, int64_t *meta, int64_t *positions, int64_t *slot_ids,
+                                  int64_t *slot_map, int32_t *cu_pages, int32_t *gather_pages, void *stream) {
+  if (n <= 0 || !lengths || !starts || !slots || page_size <= 0 || !cu_seqlens || !ends || !context_lens || !meta)
+    return DD_EINVAL;
+  if ((slot_map || gather_pages) && (!page_table || table_width <= 0)) return DD_EINVAL;
+  if (gather_pages && !cu_pages) return DD_EINVAL;
+  // 32-bit segments whose sums fit (anything larger: dd_pack_batch), and totals
+  // that are theirs
+  constexpr int64_t kMax = 0x3fffffff;
+  int64_t tokens = 0, pages = 0;
+  for (int i = 0; i < n; ++i) {
+    if (lengths[i] < 0 || starts[i] < 0) return DD_EINVAL;
+    if (lengths[i] > kMax || starts[i] > kMax || slots[i] < -kMax || slots[i] > kMax) return DD_EUNSUPPORTED;
+    tokens += lengths[i];
+    pages += (lengths[i] + starts[i] + page_size - 1) / page_size;
+    if (tokens > kMax || pages > kMax) return DD_EUNSUPPORTED;
+  }
+  if (tokens != total_tokens || (gather_pages && pages != total_pages)) return DD_EINVAL;
+  if (tokens > 0 && (!positions || !slot_ids)) return DD_EINVAL;
+  const PackOut out{cu_seqlens, ends, context_lens, meta, positions, slot_ids, slot_map, cu_pages, gather_pages};
+  PackSegs segs;
+  segs.total = n;
+  segs.tok0 = segs.page0 = 0;
+  for (segs.i0 = 0; segs.i0 < n; segs.i0 += kPackSegs) {
+    segs.n = n - segs.i0 < kPackSegs ? n - segs.i0 : kPackSegs;
+    int64_t t = 0, pg = 0;
+    for (int i = 0; i < segs.n; ++i) {
+      const int64_t len = lengths[segs.i0 + i], start = starts[segs.i0 + i];
+      segs.len[i] = (int)len;
+      segs.start[i] = (int)start;
+      segs.slot[i] = (int)slots[segs.i0 + i];
+      t += len;
+      pg += (len + start + page_size - 1) / page_size;
+    }
+    segs.tok_blocks = (int)dd_cdiv(t, kPackSegs);
+    const long grid = segs.tok_blocks + (gather_pages ? dd_cdiv(pg, kPackSegs) : 0);
+    hipLaunchKernelGGL(pack_segments_kernel, dim3((unsigned)(grid > 0 ? grid : 1)), dim3(kPackSegs), 0,
+                       (hipStream_t)stream, segs, page_table, table_rows, table_width, page_size, out);
+    DD_LAUNCH_CHECK();
+    segs.tok0 += t;
+    segs.page0 += pg;
   }
   return DD_OK;
 }

@@ -327,6 +327,36 @@ extern "C" int dd_prefill_split(const int64_t *lengths, const int64_t *starts, i
   return DD_OK;
 }
 
+extern "C" int dd_prefill_prepare(const int64_t *lengths, const int64_t *starts, int n, int heads, int kv_heads,
+                                  int dim, int dtype, int window, float scale, int workgroups, int64_t *out) {
+  if (!lengths || !starts || !out || n <= 0 || heads <= 0 || kv_heads <= 0 || heads % kv_heads) return DD_EINVAL;
+  int64_t max_len = 0, max_context = 0;
+  for (int i = 0; i < n; ++i) {
+    if (lengths[i] < 0 || starts[i] < 0 || lengths[i] + starts[i] > 0x7fffffffL) return DD_EINVAL;
+    max_len = std::max(max_len, lengths[i]);
+    max_context = std::max(max_context, lengths[i] + starts[i]);
+  }
+  const int flags = dd_prefill_flag_count(n, (int)max_len, heads, kv_heads, dim, dtype);
+  if (flags < 0) return -flags;
+  Geometry g;
+  const bool mfma = dtype != DD_F32 && scale != 0.f && geometry(dim, &g) && g.cols >= heads / kv_heads;
+  int split_tiles = 0, max_splits = 1;
+  int64_t floats = 0;
+  int rc = DD_EUNSUPPORTED;
+  if (mfma || dtype == DD_F32)
+    rc = dd_prefill_split(lengths, starts, n, heads, kv_heads, dim, dtype, window, workgroups, &split_tiles,
+                          &max_splits, &floats);
+  if (rc != DD_OK && rc != DD_EUNSUPPORTED) return rc;
+  out[0] = !mfma ? 0 : rc == DD_OK ? 1 : 2;
+  out[1] = split_tiles;
+  out[2] = max_splits;
+  out[3] = rc == DD_OK ? floats : 0;
+  out[4] = flags;
+  out[5] = max_len;
+  out[6] = max_context;
+  return DD_OK;
+}
+
 extern "C" int dd_prefill_flag_count(int n, int max_len, int heads, int kv_heads, int dim, int dtype) {
   if (n < 0 || max_len < 0 || heads <= 0 || kv_heads <= 0 || heads % kv_heads) return -DD_EINVAL;
   // only bf16 pages at the head sizes of prefill_pipe_kernel convert V to fp16

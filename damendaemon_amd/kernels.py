@@ -9,6 +9,7 @@ every call runs hand-written gfx950 HIP kernels through the C ABI in
 import ctypes
 import math
 import os
+from functools import lru_cache
 
 import torch
 
@@ -26,9 +27,14 @@ def _splits(max_context, batch_kv, dim, kv_dtype):
         if tokens <= 0 or tokens % 64:
             raise ValueError('DAMENDAEMON_AMD_SPLIT_TOKENS must be a positive multiple of 64')
         return -(-int(max_context) // tokens), tokens
+    return _policy(int(max_context), int(batch_kv), int(dim), DTYPE_CODES[kv_dtype])
+
+
+@lru_cache(maxsize=1024)
+def _policy(max_context, batch_kv, dim, kv_code):
+    """The library's split policy, a pure function of these numbers."""
     tokens = ctypes.c_int(0)
-    splits = _native.library().dd_decode_splits_for(int(max_context), int(batch_kv), int(dim), DTYPE_CODES[kv_dtype],
-                                                     ctypes.byref(tokens))
+    splits = _native.library().dd_decode_splits_for(max_context, batch_kv, dim, kv_code, ctypes.byref(tokens))
     if splits <= 0:
         raise ValueError('invalid decode geometry')
     return splits, tokens.value
@@ -148,29 +154,48 @@ class DecodeLaunch:
         if out is not None and (out.shape != query.shape or out.dtype != query.dtype or not out.is_contiguous()):
             raise ValueError('out must be a contiguous tensor shaped and typed like the query')
         self.out = torch.empty_like(query) if out is None else out
-        if splits > 1:
-            self.partial = torch.empty((batch * heads, splits, dim), device=query.device, dtype=torch.float32)
-            self.lse = torch.empty((batch * heads, splits), device=query.device, dtype=torch.float32)
-        else:
-            self.partial = self.lse = None
+        # partials (batch * heads, splits, dim), then log-sum-exps (batch * heads, splits)
+        rows = batch * heads * splits if splits > 1 else 0
+        scratch = torch.empty(rows * (dim + 1), device=query.device, dtype=torch.float32) if rows else None
+        partial = lse = None
+        if rows:
+            partial = scratch.data_ptr()
+            lse = partial + 4 * rows * dim
         self.splits, self.split_tokens = splits, split_tokens
+        self._scratch, self._partial_shape = scratch, (batch * heads, splits, dim)
         # keep every tensor argument alive as long as the launch object
         self._keep = (query, cache_k, cache_v, positions, slots, page_table, k_scale, v_scale, alibi,
                       relative_bias, sinks)
-        self._device = query.device
+        self._index = query.get_device()
+        table_rows, table_width = (0, 0) if page_table is None else page_table.shape
         self._args = (
-            ptr(query), DTYPE_CODES[query.dtype], ptr(cache_k), ptr(cache_v), DTYPE_CODES[cache_k.dtype],
-            ptr(k_scale), ptr(v_scale), group,
-            ptr(positions), ptr(slots), ptr(page_table),
-            0 if page_table is None else page_table.shape[0], 0 if page_table is None else page_table.shape[1],
+            query.data_ptr(), DTYPE_CODES[query.dtype], cache_k.data_ptr(), cache_v.data_ptr(),
+            DTYPE_CODES[cache_k.dtype], ptr(k_scale), ptr(v_scale), group,
+            positions.data_ptr(), ptr(slots), ptr(page_table), table_rows, table_width,
             batch, heads, kv_heads, dim, page_size, capacity, int(window or 0),
             float(dim ** -.5 if scale is None else scale),
             ptr(alibi), ptr(relative_bias), buckets,
             math.log(relative_max_distance / (buckets // 2)) if buckets else 1.0,
-            ptr(sinks), ptr(self.out), ptr(self.partial), ptr(self.lse), splits, split_tokens)
+            ptr(sinks), self.out.data_ptr(), partial, lse, splits, split_tokens)
+
+    @property
+    def partial(self):
+        """The split partials (batch * heads, splits, dim), or None with one split."""
+        if self._scratch is None:
+            return None
+        rows, splits, dim = self._partial_shape
+        return self._scratch[:rows * splits * dim].view(rows, splits, dim)
+
+    @property
+    def lse(self):
+        """Their log-sum-exps (batch * heads, splits), or None with one split."""
+        if self._scratch is None:
+            return None
+        rows, splits, dim = self._partial_shape
+        return self._scratch[rows * splits * dim:].view(rows, splits)
 
     def _call(self, name):
-        call(name, *self._args, ctypes.c_void_p(torch.cuda.current_stream(self._device).cuda_stream))
+        call(name, *self._args, _native.stream_on(self._index))
 
     def run(self):
         self._call('dd_decode_attention')
@@ -210,8 +235,10 @@ def rope_batch(qkv, cos, sin, positions, slots, cache_k, cache_v, heads, q_norm=
         raise ValueError('q_norm and k_norm go together')
     if norm is not None and (q_norm.dtype != k_norm.dtype or q_norm.numel() != dim or k_norm.numel() != dim):
         raise ValueError('norm weights must be (dim,) of one dtype')
-    positions = positions.to(torch.int64)
-    slots = slots.to(torch.int64)
+    if positions.dtype != torch.int64:
+        positions = positions.to(torch.int64)
+    if slots.dtype != torch.int64:
+        slots = slots.to(torch.int64)
     if page_table is not None and (page_table.dtype != torch.int32 or not page_table.is_contiguous()):
         raise ValueError('page table must be a contiguous int32 matrix')
     query = torch.empty((tokens, heads, 1, dim), device=qkv.device, dtype=qkv.dtype)

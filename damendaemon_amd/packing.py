@@ -3,8 +3,8 @@
 ``pack_batch`` replaces the host-side packing of damendaemon/paged.py:149-159
 (flat ``positions``/``slot_ids`` built by list comprehensions), the
 ``accumulate(lengths)`` segment ends of paged.py:118-120 and the physical
-slot computation of kernels.py:279-281: the host uploads one (3, n) int64
-array of (length, start, slot) per segment and the GPU expands it.
+slot computation of kernels.py:279-281: the (length, start, slot) of every
+segment travel in the launch's arguments and the GPU expands them.
 """
 from dataclasses import dataclass
 
@@ -48,28 +48,42 @@ def pack_batch(lengths, starts, slots, page_table=None, page_size=16, device='cu
         raise ValueError('invalid packing request')
     n = host.shape[1]
     lengths, starts, slots = host.tolist()
-    total = int(host[0].sum())
-    pages = int(((host[0] + host[1] + (page_size - 1)) // page_size).sum())
+    total = sum(lengths)
+    with_table = page_table is not None
+    gather = gather and with_table
+    pages = sum([(a + b + (page_size - 1)) // page_size for a, b in zip(lengths, starts)]) if gather else 0
     dev = torch.device(device)
-    meta = torch.from_numpy(host)
-    meta = _native.upload(meta, dev) if dev.type == 'cuda' else meta.to(dev)
-    _native.require_device(meta, page_table)
-    if page_table is not None and (page_table.dtype != torch.int32 or not page_table.is_contiguous()):
+    if dev.type != 'cuda':
+        raise ValueError('damendaemon_amd kernels need tensors on the GPU (there is no CPU path)')
+    _native.refuse_capture()
+    _native.require_device(page_table)
+    if with_table and (page_table.dtype != torch.int32 or not page_table.is_contiguous()):
         raise ValueError('page table must be a contiguous int32 matrix')
-    i64 = dict(dtype=torch.int64, device=dev)
-    out = PackedBatch(
-        cu_seqlens=torch.empty(n + 1, **i64), ends=torch.empty(n, **i64), context_lens=torch.empty(n, **i64),
-        positions=torch.empty(total, **i64), slot_ids=torch.empty(total, **i64),
-        slot_map=torch.empty(total, **i64) if page_table is not None else None,
-        cu_pages=torch.empty(n + 1, dtype=torch.int32, device=dev) if page_table is not None and gather else None,
-        gather_pages=torch.empty(pages, dtype=torch.int32, device=dev) if page_table is not None and gather else None,
-        lengths=lengths, starts=starts, slots=slots, total_tokens=total, page_size=page_size)
-    call('dd_pack_batch', ptr(meta[0]), ptr(meta[1]), ptr(meta[2]), n, total, pages if out.gather_pages is not None else 0,
-         ptr(page_table), 0 if page_table is None else page_table.shape[0],
-         0 if page_table is None else page_table.shape[1], page_size,
-         ptr(out.cu_seqlens), ptr(out.ends), ptr(out.context_lens), ptr(out.positions), ptr(out.slot_ids),
-         ptr(out.slot_map), ptr(out.cu_pages), ptr(out.gather_pages), _native.stream_of(meta))
-    out._meta = meta  # keep the uploaded metadata alive until the kernels ran
+    # one allocation for the int64 outputs and one for the int32 ones
+    sizes = [n + 1, n, n, 3 * n, total, total, total if with_table else 0]
+    buffer = torch.empty(sum(sizes), dtype=torch.int64, device=dev)
+    cu_seqlens, ends, context_lens, meta, positions, slot_ids, slot_map = buffer.split(sizes)
+    cu_pages, gather_pages = (torch.empty(n + 1 + pages, dtype=torch.int32, device=dev).split([n + 1, pages])
+                              if gather else (None, None))
+    meta = meta.view(3, n)
+    out = PackedBatch(cu_seqlens, ends, context_lens, positions, slot_ids, slot_map if with_table else None, cu_pages,
+                      gather_pages, lengths, starts, slots, total, page_size)
+    table_args = (ptr(page_table), *(page_table.shape if with_table else (0, 0)), page_size)
+    results = (ptr(positions), ptr(slot_ids), ptr(out.slot_map), ptr(cu_pages), ptr(gather_pages),
+               _native.stream_of(buffer))
+    source = host.ctypes.data
+    code = _native.UNSUPPORTED
+    if n:
+        code = _native.status('dd_pack_batch_host', source, source + 8 * n, source + 16 * n, n, total, pages, *table_args,
+                              ptr(cu_seqlens), ptr(ends), ptr(context_lens), ptr(meta), *results)
+    if code == _native.UNSUPPORTED:   # no segments, or values past 30 bits
+        meta.copy_(_native.upload(torch.from_numpy(host), buffer.device))
+        first = ptr(meta)
+        call('dd_pack_batch', first, first + 8 * n, first + 16 * n, n, total, pages, *table_args, ptr(cu_seqlens),
+             ptr(ends), ptr(context_lens), *results)
+    elif code:
+        _native.check('dd_pack_batch_host', code)
+    out._meta, out._host = meta, host
     return out
 
 
@@ -86,7 +100,8 @@ def store_kv_pages(key, value, slot_map, cache_k, cache_v, k_scale=None, v_scale
             or cache_v.shape != cache_k.shape or not cache_k.is_contiguous() or not cache_v.is_contiguous()):
         raise ValueError('incompatible K/V page write shapes')
     _native.require_device(key, value, slot_map, cache_k, cache_v)
-    slot_map = slot_map.to(torch.int64)
+    if slot_map.dtype != torch.int64:
+        slot_map = slot_map.to(torch.int64)
     if cache_k.dtype == torch.int8:
         if k_scale is None or v_scale is None or k_scale.shape[:-1] != cache_k.shape[:-1] or dim % k_scale.shape[-1]:
             raise ValueError('int8 pages need fp16 scales (..., page, dim/group)')

@@ -6,8 +6,8 @@ with a lower-right causal mask (qwen2.py:756-770), and decodes through
 ``kernels.attention`` in a separate forward pass (scheduler.py:822-873).
 Here one packed token buffer (from ``packing.pack_batch``) is attended in
 place: multi-token segments by the paged MFMA prefill kernel, the trailing
-run of single-token segments by the split-KV decode kernel.  Both read the
-pages directly; nothing is gathered.
+run of single-token segments by the split-KV decode kernel, one after the
+other.  Both read the pages directly; nothing is gathered.
 """
 import ctypes
 import math
@@ -36,14 +36,6 @@ def _check(query, cache_k, cache_v, page_table):
     return query
 
 
-def _has_mfma_geometry(dim, group):
-    """Whether the 16-bit MFMA prefill kernels take this head size and number
-    of query heads per KV head (then the call carries a workgroup plan)."""
-    cols, keys = ctypes.c_int(0), ctypes.c_int(0)
-    ok = _native.library().dd_prefill_geometry(int(dim), ctypes.byref(cols), ctypes.byref(keys)) == 0
-    return ok and cols.value >= group
-
-
 def prefill_plan(lengths, starts, heads, kv_heads, dim, window=0, slots=None, workgroups=0):
     """Schedule of the prefill kernel for these segments: a host int32 array
     (entries, 8), each row (item or -1, first packed token, length, start,
@@ -61,17 +53,18 @@ def prefill_plan(lengths, starts, heads, kv_heads, dim, window=0, slots=None, wo
     if lengths.shape != starts.shape or lengths.shape != slots.shape or lengths.ndim != 1:
         raise ValueError('lengths, starts and slots must be matching 1-D sequences')
     lib = _native.library()
-    args = (lengths.ctypes.data_as(ctypes.c_void_p), starts.ctypes.data_as(ctypes.c_void_p),
-            slots.ctypes.data_as(ctypes.c_void_p), len(lengths), heads, kv_heads, dim, int(window or 0),
+    args = (lengths.ctypes.data, starts.ctypes.data, slots.ctypes.data, len(lengths), heads, kv_heads, dim, int(window or 0),
             int(workgroups))
-    need = lib.dd_prefill_plan(*args, None, 0)
-    if need < 0:
-        raise _native.NativeError(f'dd_prefill_plan failed: {lib.dd_error_string(-need).decode()} ({-need})')
-    plan = np.empty((max(need, 1), PLAN_INTS), dtype=np.int32)
-    got = lib.dd_prefill_plan(*args, plan.ctypes.data_as(ctypes.c_void_p), len(plan))
-    if got != need:
-        raise _native.NativeError('dd_prefill_plan returned an inconsistent length')
-    return plan[:need]
+    # (a guess that holds for balanced schedules first: the length is only known once the schedule is)
+    rows = 512 + 2 * kv_heads * int((lengths // 32 + 1).sum()) if workgroups > 0 else 0
+    while True:
+        plan = np.empty((max(rows, 1), PLAN_INTS), dtype=np.int32)
+        need = lib.dd_prefill_plan(*args, plan.ctypes.data, rows)
+        if need < 0:
+            raise _native.NativeError(f'dd_prefill_plan failed: {lib.dd_error_string(-need).decode()} ({-need})')
+        if need <= rows:
+            return plan[:need]
+        rows = need
 
 
 PLAN_INTS = 8   # DD_PREFILL_PLAN_INTS
@@ -84,10 +77,9 @@ def prefill_split(lengths, starts, heads, kv_heads, dim, dtype, window, device):
     lengths = np.ascontiguousarray(lengths, dtype=np.int64)
     starts = np.ascontiguousarray(starts, dtype=np.int64)
     tiles, splits, floats = ctypes.c_int(0), ctypes.c_int(1), ctypes.c_int64(0)
-    code = _native.library().dd_prefill_split(
-        lengths.ctypes.data_as(ctypes.c_void_p), starts.ctypes.data_as(ctypes.c_void_p), len(lengths), heads, kv_heads,
-        dim, DTYPE_CODES[dtype], int(window or 0), _cu_count(device), ctypes.byref(tiles), ctypes.byref(splits),
-        ctypes.byref(floats))
+    code = _native.status('dd_prefill_split', lengths.ctypes.data, starts.ctypes.data, len(lengths), heads, kv_heads, dim,
+                          DTYPE_CODES[dtype], int(window or 0), _cu_count(device), ctypes.byref(tiles),
+                          ctypes.byref(splits), ctypes.byref(floats))
     return None if code else (tiles.value, splits.value, floats.value)
 
 
@@ -107,11 +99,17 @@ def prefill_attention(query, cache_k, cache_v, packed, page_table, window=0, sca
 
 def prepare_prefill(query, cache_k, cache_v, packed, page_table, window=0, scale=None, out=None, segments=None,
                     flags=None):
-    """Validate a prefill call, compute and upload its workgroup plan, and
-    return a ``PrefillLaunch`` whose ``run()`` only enqueues the kernels
+    """Validate a prefill call, size its workspaces, upload its workgroup plan
+    when it has more work items than the GPU has CUs, and return a
+    ``PrefillLaunch`` whose ``run()`` only enqueues the kernels
     (arguments and errors as ``prefill_attention``)."""
-    q = _check(query, cache_k, cache_v, page_table)
+    return _prepare_prefill(_check(query, cache_k, cache_v, page_table), cache_k, cache_v, packed, page_table, window,
+                            scale, out, segments, flags)
+
+
+def _prepare_prefill(q, cache_k, cache_v, packed, page_table, window, scale, out, segments, flags):
     T, H, D = q.shape
+    capacity, KH, page, _ = cache_k.shape
     scale = float(D ** -.5 if scale is None else scale)
     if not math.isfinite(scale):
         raise ValueError('prefill attention needs a finite scale')
@@ -122,44 +120,42 @@ def prepare_prefill(query, cache_k, cache_v, packed, page_table, window=0, scale
                 or not out.is_contiguous()):
             raise ValueError('out must be a contiguous tensor of the query dtype, device and size')
         out = out.view(q.shape)
-    a, b = segments if segments is not None else (0, len(packed.lengths))
+    count = len(packed.lengths)
+    a, b = segments if segments is not None else (0, count)
+    a, b, _ = slice(a, b).indices(count)
     if b <= a:
         return PrefillLaunch(out, None)
-    max_len = max(packed.lengths[a:b])
-    max_context = max(s + n for s, n in zip(packed.starts[a:b], packed.lengths[a:b]))
-    plan_dev, plan_len, scratch = None, 0, None
-    split = None
-    mfma = q.dtype != torch.float32 and scale != 0.0 and _has_mfma_geometry(D, H // cache_k.shape[1])
-    if mfma:
+    n, window, code = b - a, int(window or 0), DTYPE_CODES[q.dtype]
+    host = getattr(packed, '_host', None)
+    if host is None:
+        host = np.array((packed.lengths, packed.starts, packed.slots), dtype=np.int64)
+    first = host.ctypes.data + 8 * a
+    sizes = (ctypes.c_int64 * 7)()
+    call('dd_prefill_prepare', first, first + 8 * count, n, H, KH, D, code, window, scale, _cu_count(q.device), sizes)
+    schedule, split_tiles, max_splits, floats, n_flags, max_len, max_context = sizes
+    if schedule:
         _native.refuse_capture()
-    if mfma or q.dtype == torch.float32:
-        split = prefill_split(packed.lengths[a:b], packed.starts[a:b], H, cache_k.shape[1], D, q.dtype, window,
-                              q.device)
-    split_tiles, max_splits, floats = split or (0, 1, 0)
-    if floats:
-        scratch = torch.empty(floats, dtype=torch.float32, device=q.device)
-    if mfma and split is None:
+    plan_dev, plan_len = None, 0
+    if schedule == 2:
         # more work items than CUs: the MFMA kernel's XCD-balanced workgroup
         # order (with fewer there is nothing to order, and nothing to upload)
-        plan = prefill_plan(packed.lengths[a:b], packed.starts[a:b], H, cache_k.shape[1], D, window,
-                            packed.slots[a:b], _persistent_workgroups(q.device, D))
+        plan = prefill_plan(host[0, a:b], host[1, a:b], H, KH, D, window, host[2, a:b],
+                            _persistent_workgroups(q.device, D))
         if len(plan) == 0:
             return PrefillLaunch(out, None)
         plan_dev = _native.upload(torch.from_numpy(plan), q.device)
         plan_len = len(plan) // int(plan[0, 5])     # workgroups
-    n_flags = prefill_flag_count(b - a, max_len, H, cache_k.shape[1], D, q.dtype)
+    scratch = torch.empty(floats, dtype=torch.float32, device=q.device) if floats else None
     # per-item exactness flags of the bf16 kernel (written by the kernel itself)
     if flags is not None:
         if flags.dtype != torch.int32 or flags.device != q.device or flags.numel() < n_flags:
             raise ValueError(f'flags must be int32 on the query device with at least {n_flags} entries')
     elif n_flags:
         flags = torch.empty(n_flags, dtype=torch.int32, device=q.device)
-    args = (ptr(q), ptr(cache_k), ptr(cache_v), DTYPE_CODES[q.dtype],
-            ptr(packed.cu_seqlens[a:]), ptr(packed.context_lens[a:]), ptr(packed._meta[2, a:]), b - a, max_len,
-            max_context, ptr(page_table), page_table.shape[0], page_table.shape[1], H, cache_k.shape[1], D,
-            cache_k.shape[2], cache_k.shape[0], int(window or 0), scale,
-            ptr(plan_dev), plan_len, ptr(flags), ptr(out), split_tiles, max_splits, ptr(scratch),
-            0 if scratch is None else scratch.numel())
+    args = (q.data_ptr(), cache_k.data_ptr(), cache_v.data_ptr(), code, packed.cu_seqlens.data_ptr() + 8 * a,
+            packed.context_lens.data_ptr() + 8 * a, packed._meta.data_ptr() + 8 * (2 * count + a), n, max_len,
+            max_context, page_table.data_ptr(), *page_table.shape, H, KH, D, page, capacity, window, scale,
+            ptr(plan_dev), plan_len, ptr(flags), out.data_ptr(), split_tiles, max_splits, ptr(scratch), floats)
     return PrefillLaunch(out, args, keep=(q, cache_k, cache_v, packed, page_table, plan_dev, flags, scratch))
 
 
@@ -170,6 +166,7 @@ class PrefillLaunch:
 
     def __init__(self, out, args, keep=()):
         self.out, self._args, self._keep = out, args, keep
+        self._index = out.get_device()
 
     def run(self):
         return self.phase(3)
@@ -178,8 +175,7 @@ class PrefillLaunch:
         """Enqueue one launch of the call: 1 the attention kernel, 2 the exact
         re-run of the items the bf16 kernel flagged (both together = run())."""
         if self._args is not None:
-            call('dd_prefill_attention_split', *self._args, int(which),
-                 ctypes.c_void_p(torch.cuda.current_stream(self.out.device).cuda_stream))
+            call('dd_prefill_attention_split', *self._args, int(which), _native.stream_on(self._index))
         return self.out
 
 
@@ -217,7 +213,13 @@ def prefill_flag_count(segments, max_len, heads, kv_heads, dim, dtype):
 def ragged_attention(query, cache_k, cache_v, packed, page_table, window=0, scale=None):
     """Mixed batch: the trailing single-token segments decode, the rest prefill.
 
-    Returns (T, H, D) in the query dtype.
+    Returns (T, H, D) in the query dtype.  The prefill chunks run before the
+    decode rows on the caller's stream.  (Side by side on two streams they gain
+    nothing: a prefill workgroup fills a CU's LDS and registers, so a decode
+    workgroup only gets onto CUs that have none, and the events between the
+    streams cost the host more than the tails that overlap.  8 chunks of 512
+    tokens and 120 rows, with pack and rope: 571-588 us on two streams,
+    548-552 on one.)
     """
     q = _check(query, cache_k, cache_v, page_table)
     T, H, D = q.shape
@@ -227,38 +229,11 @@ def ragged_attention(query, cache_k, cache_v, packed, page_table, window=0, scal
     first_decode = n
     while first_decode > 0 and lengths[first_decode - 1] == 1:
         first_decode -= 1
-    t_decode = sum(lengths[:first_decode])
-
-    def decode():
-        rows = slice(t_decode, T)
+    if first_decode > 0:
+        _prepare_prefill(q, cache_k, cache_v, packed, page_table, window, scale, out, (0, first_decode), None).run()
+    if first_decode < n:
+        rows = slice(sum(lengths[:first_decode]), T)
         kernels.prepare_attention(q[rows].unsqueeze(2), cache_k, cache_v, packed.positions[rows],
                                   packed.slot_ids[rows], window=window, scale=scale, page_table=page_table,
                                   out=out[rows].unsqueeze(2)).run()
-
-    if first_decode > 0 and first_decode < n:
-        # The decode rows (HBM-bound) run on a side stream beside the prefill
-        # chunks (matrix cores): C4 526 us vs 586 us one after the other.  The
-        # two write disjoint rows of `out`; the caller's stream waits for both.
-        main = torch.cuda.current_stream(q.device)
-        side = _side_stream(q.device)
-        side.wait_stream(main)
-        with torch.cuda.stream(side):
-            decode()
-        prefill_attention(q, cache_k, cache_v, packed, page_table, window, scale, out, (0, first_decode))
-        main.wait_stream(side)
-    elif first_decode > 0:
-        prefill_attention(q, cache_k, cache_v, packed, page_table, window, scale, out, (0, first_decode))
-    elif first_decode < n:
-        decode()
     return out
-
-
-_SIDE_STREAMS = {}
-
-
-def _side_stream(device):
-    """One extra stream per device, default priority, for the decode half of a mixed batch."""
-    key = torch.device(device).index
-    if key not in _SIDE_STREAMS:
-        _SIDE_STREAMS[key] = torch.cuda.Stream(device=device)
-    return _SIDE_STREAMS[key]

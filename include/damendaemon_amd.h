@@ -199,6 +199,23 @@ int dd_pack_batch(const int64_t *lengths, const int64_t *starts,
                   int32_t *cu_pages, int32_t *gather_pages, void *stream);
 
 /*
+ * dd_pack_batch for segments held on the HOST (the three arrays are read
+ * before the call returns): they travel in the launch's arguments, so that
+ * nothing is uploaded.  meta (int64, device, 3 x n) receives the segments'
+ * lengths, starts and slots.  n >= 1.  Returns DD_EUNSUPPORTED for values or
+ * sums past 30 bits (upload them and call dd_pack_batch).
+ */
+int dd_pack_batch_host(const int64_t *lengths, const int64_t *starts,
+                       const int64_t *slots, int n, int64_t total_tokens,
+                       int64_t total_pages, const int32_t *page_table,
+                       int table_rows, int table_width, int page_size,
+                       int64_t *cu_seqlens, int64_t *ends,
+                       int64_t *context_lens, int64_t *meta,
+                       int64_t *positions, int64_t *slot_ids,
+                       int64_t *slot_map, int32_t *cu_pages,
+                       int32_t *gather_pages, void *stream);
+
+/*
  * Write new K/V rows (tokens, kv_heads, dim) into their page slots
  * (slot_map from dd_pack_batch; negative entries are skipped): the page
  * write half of damendaemon/kernels.py:312-319 without the rotation.
@@ -346,6 +363,19 @@ int dd_prefill_split(const int64_t *lengths, const int64_t *starts, int n,
                      int heads, int kv_heads, int dim, int dtype, int window,
                      int workgroups, int *split_tiles, int *max_splits,
                      int64_t *scratch_floats);
+
+/*
+ * Everything a caller of dd_prefill_attention_split sizes its call with, from
+ * the HOST segments (n >= 1), in one call: out (int64, 7) receives
+ *   0  the schedule: 0 no 16-bit MFMA kernel (no plan), 1 16-bit without a
+ *      plan, 2 16-bit with a plan (dd_prefill_plan)
+ *   1, 2, 3  split_tiles, max_splits and scratch_floats of dd_prefill_split
+ *   4  dd_prefill_flag_count
+ *   5, 6  the longest segment and the longest start + length
+ */
+int dd_prefill_prepare(const int64_t *lengths, const int64_t *starts, int n,
+                       int heads, int kv_heads, int dim, int dtype, int window,
+                       float scale, int workgroups, int64_t *out);
 
 /*
  * Entries of dd_prefill_attention's flags workspace for these arguments (0

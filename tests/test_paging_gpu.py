@@ -324,3 +324,32 @@ def test_rope_lane_layouts(dim, rd, dtype, precise):
                                             page_table=wide)
         for have, want in ((q, eq), (k, ek), (v, ev), (dk, eck[:cap]), (dv, ecv[:cap])):
             assert torch.equal(have.cpu(), want)
+
+
+@pytest.mark.parametrize('n', [1, 255, 256, 257, 600])
+@pytest.mark.parametrize('big', [0, 1 << 40])
+def test_pack_segment_launches(n, big):
+    """Segments in the launch's arguments, 256 at a time (empty ones at the edges of a launch), and
+    values past 30 bits, which are uploaded; the segments' copies that the prefill kernels read."""
+    rng = random.Random(n)
+    lengths = [rng.choice([0, 1, 1, 37]) for _ in range(n)]
+    starts = [rng.choice([0, 5, 300]) for _ in range(n)]
+    lengths[-1], starts[0] = 0 if n > 1 else 3, starts[0] + big
+    if n > 256:
+        lengths[255] = lengths[256] = 0
+    slots = [rng.randrange(50) for _ in range(n)]
+    table = torch.arange(50 * 30, dtype=torch.int32).reshape(50, 30)
+    got = packing.pack_batch(lengths, starts, slots, table.to(DEV), gather=not big)
+    want_map = []
+    for length, start, slot in zip(lengths, starts, slots):
+        for p in range(start, start + length):
+            want_map.append((int(table[slot, p // 16]) if p // 16 < 30 else -1) * 16 + p % 16)
+    assert got.slot_map.cpu().tolist() == want_map
+    ends = torch.tensor(lengths).cumsum(0)
+    assert got.cu_seqlens.cpu().tolist() == [0] + ends.tolist() and got.ends.cpu().tolist() == (ends - 1).tolist()
+    assert got.context_lens.cpu().tolist() == [a + b for a, b in zip(starts, lengths)]
+    assert got._meta.cpu().tolist() == [lengths, starts, slots]
+    if not big:
+        pages = [-(-(a + b) // 16) for a, b in zip(starts, lengths)]
+        assert got.cu_pages.cpu().tolist() == [0] + torch.tensor(pages).cumsum(0).tolist()
+        assert got.gather_pages.cpu().tolist() == [int(table[s, k]) for s, c in zip(slots, pages) for k in range(c)]
