@@ -10,10 +10,9 @@
 //     denominator once (kernels.py:168-176, 198-206);
 //   * long contexts are split; splits are combined by log-sum-exp.
 //
-// The streamed kernels of decode_stream.h take every 16-bit and fp32 case,
-// int8 pages with one scale per row at every head size and int8 pages with
-// group-32 scales at 64, 128 and 256; decode_kernel below, the general
-// kernel, serves the remaining int8 cases.
+// The streamed kernels of decode_stream.h take every 16-bit and fp32 case and
+// int8 pages with one scale per row or per 32 channels; decode_kernel below,
+// the general kernel, serves the remaining int8 groupings.
 //
 // General kernel (not a translation of the Triton kernel):
 //   * one workgroup = one (sequence, KV head, split); its 4 wavefronts take
@@ -716,7 +715,7 @@ namespace dd_decode {
 // pages at every head size up to 256 that is a multiple of 8 (in the
 // smallest streamed layout that holds it), int8 pages with one scale per row
 // at every head size that is a multiple of 16 (the same way) and int8 pages
-// with group-32 scales at D = 64, 128, 256 take the streamed kernels
+// with group-32 scales at every multiple of 32 take the streamed kernels
 // (decode_stream.h), any number of query heads per KV head; the other int8
 // groupings take decode_kernel.
 // LDS layout of the streamed 16-bit / fp32 kernels for head size D: the
@@ -775,21 +774,29 @@ int dispatch_d(const DecodeParams &p0, int D, hipStream_t s, int phase) {
       } else if (p.group == 32) {
         switch (D) {
           case 64: return launch_stream_i8<QT, 64, 2, DD_STREAM_I8_NB64, DD_STREAM_I8_NW64>(p, s, phase);
+          // (96 to 224 in the next layout up: the general kernel has registers
+          // for two query heads per KV head and spills from four on, 111 us
+          // for 48 sequences of 55 keys and 4 heads at 96, 12.8 here; 64 of up to 8,192 keys 833 -> 119 us)
+          case 96: return launch_stream_i8<QT, 128, 3, DD_STREAM_NB128G, DD_STREAM_I8_NW128>(p, s, phase);
           case 128: return launch_stream_i8<QT, 128, 4, DD_STREAM_NB128G, DD_STREAM_I8_NW128>(p, s, phase);
+          case 160: return launch_stream_i8<QT, 256, 5, DD_STREAM_I8_NB256, DD_STREAM_I8_NW256>(p, s, phase);
+          case 192: return launch_stream_i8<QT, 256, 6, DD_STREAM_I8_NB256, DD_STREAM_I8_NW256>(p, s, phase);
+          case 224: return launch_stream_i8<QT, 256, 7, DD_STREAM_I8_NB256, DD_STREAM_I8_NW256>(p, s, phase);
           case 256: return launch_stream_i8<QT, 256, 8, DD_STREAM_I8_NB256, DD_STREAM_I8_NW256>(p, s, phase);
           default: break;
         }
       }
     }
   }
-  // the general kernel: the smallest layout of 64, 96, 128, 256 dims that
-  // holds the head size (a multiple of 8, of 16 for int8 pages: whole
-  // 16-byte loads)
-  if (D <= 0 || D % (KVT == DD_I8 ? 16 : 8) || D > 256) return DD_EUNSUPPORTED;
-  if (D <= 64) return dispatch_g<KVT, QT, 64>(p0, s, phase);
-  if (D <= 96) return dispatch_g<KVT, QT, 96>(p0, s, phase);
-  if (D <= 128) return dispatch_g<KVT, QT, 128>(p0, s, phase);
-  return dispatch_g<KVT, QT, 256>(p0, s, phase);
+  // the general kernel: int8 pages with scale groups between 32 channels and
+  // the whole head (64 of 128, 192 or 256; 96 of 192; 128 of 256), in layouts
+  // of 128 and 256 dims
+  if constexpr (KVT == DD_I8) {
+    if (D <= 0 || D % 16 || D > 256) return DD_EUNSUPPORTED;
+    if (D <= 128) return dispatch_g<KVT, QT, 128>(p0, s, phase);
+    return dispatch_g<KVT, QT, 256>(p0, s, phase);
+  }
+  return DD_EUNSUPPORTED;
 }
 
 }  // namespace dd_decode

@@ -3,8 +3,8 @@
 // 160, 192, 224 and 256 dims; a smaller head size takes the smallest layout
 // that holds it, its rows of the real length in memory and the layout's
 // extra dims zeros), and for int8 pages (stream_i8_kernel below: one scale
-// per row at every head size that is a multiple of 16, in layouts of 64, 128
-// and 256 dims; group-32 scales at 64, 128 and 256).
+// per row at every head size that is a multiple of 16, group-32 scales at
+// every multiple of 32, in layouts of 64, 128 and 256 dims).
 //
 // Same contract as decode_kernel (the reference's `_attention`,
 // damendaemon/kernels.py:134-187): one query row per sequence, keys
@@ -779,9 +779,13 @@ __global__ __launch_bounds__(64 * NW) void stream_i8_kernel(DecodeParams p) {
   constexpr int CPR16 = ROWB / 16;
   constexpr int NC = D / 32;
   constexpr int MD = D / 16;
+  // k-steps and O^T blocks that hold channels: with group-32 scales the head
+  // size is 32 NG (known here), with one scale per row any up to D
+  constexpr int NCR = NG == 1 ? NC : NG;
+  constexpr int MDR = NG == 1 ? MD : 2 * NG;
   constexpr int DP = D + 4;
   static_assert(IPC >= 1 && LPP * NB < 64 && NB >= 2 && NB <= 4, "vmcnt range, unrolled steps");
-  static_assert(NG == 1 || NG == NC, "one scale per row or per 32 channels");
+  static_assert(NG <= NC, "one scale per row or per 32 channels");
   static_assert((NB - 1) * STAGE + SOFF0 + 4 * SCB < 65536, "ds offset range");
   static_assert(NW * 16 * DP * 4 <= NW * NB * STAGE, "epilogue buffer fits the ring");
 
@@ -821,8 +825,7 @@ __global__ __launch_bounds__(64 * NW) void stream_i8_kernel(DecodeParams p) {
   const long head0 = (long)b * p.H + (long)kh * p.G + gofs;
   const bool col_on = n16 < G;
 
-  // The head size DR may be below the layout's D (one scale per row only):
-  // rows are DR bytes in memory, the layout's dims DR .. D-1 are zero
+  // The head size DR may be below the layout's D: rows are DR bytes in memory, the layout's dims DR .. D-1 are zero
   // queries and zero bytes in LDS, and they are never stored.
   const int DR = p.DR;
   u32x4 qa[NC];
@@ -983,15 +986,15 @@ __global__ __launch_bounds__(64 * NW) void stream_i8_kernel(DecodeParams p) {
   auto consume = [&](int i, auto stage_tag) __attribute__((always_inline)) {
     constexpr int SO = decltype(stage_tag)::value * STAGE;
     const int t0 = (pg_first + 2 * (first + i * NW)) * 16;  // first key of the pair
-    u32x2 k8[2][NC];
-    u32x2 v8[MD];
+    u32x2 k8[2][NCR];
+    u32x2 v8[MDR];
     u32x2 ks8[2][NG], vs8[2][NG];
 #pragma unroll
     for (int ch = 0; ch < 2; ++ch)
 #pragma unroll
-      for (int c = 0; c < NC; ++c) k8[ch][c] = lds_read_b64<SO>(k_addr[ch][c]);
+      for (int c = 0; c < NCR; ++c) k8[ch][c] = lds_read_b64<SO>(k_addr[ch][c]);
 #pragma unroll
-    for (int md = 0; md < MD; ++md) v8[md] = lds_read_tr8<SO>(v_addr[md]);
+    for (int md = 0; md < MDR; ++md) v8[md] = lds_read_tr8<SO>(v_addr[md]);
 #pragma unroll
     for (int ch = 0; ch < 2; ++ch)
 #pragma unroll
@@ -1003,7 +1006,7 @@ __global__ __launch_bounds__(64 * NW) void stream_i8_kernel(DecodeParams p) {
 #pragma unroll
     for (int ch = 0; ch < 2; ++ch) {
 #pragma unroll
-      for (int c = 0; c < NC; ++c) after_wait(k8[ch][c]);
+      for (int c = 0; c < NCR; ++c) after_wait(k8[ch][c]);
 #pragma unroll
       for (int g = 0; g < NG; ++g) {
         after_wait(ks8[ch][g]);
@@ -1011,7 +1014,7 @@ __global__ __launch_bounds__(64 * NW) void stream_i8_kernel(DecodeParams p) {
       }
     }
 #pragma unroll
-    for (int md = 0; md < MD; ++md) after_wait(v8[md]);
+    for (int md = 0; md < MDR; ++md) after_wait(v8[md]);
     issue(i + NB, decltype(stage_tag)::value);
 
     // scale of key 4kg + e of chunk ch, channel group g (fp16 at index e NG + g)
@@ -1064,7 +1067,7 @@ __global__ __launch_bounds__(64 * NW) void stream_i8_kernel(DecodeParams p) {
         }
       } else {
 #pragma unroll
-        for (int c = 0; c < NC; ++c) {
+        for (int c = 0; c < NG; ++c) {
           const f32x4 part = mfma16x16x32<DD_F16>(widen_i8x8_off(k8[ch][c]), qh[c], f32x4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
           for (int e = 0; e < 4; ++e) sacc[e] += scale_of(ks8, ch, e, c) * (part[e] - qoff[c]);
@@ -1098,11 +1101,17 @@ __global__ __launch_bounds__(64 * NW) void stream_i8_kernel(DecodeParams p) {
           // lies in [2^(E-15), 2^(E-14)) (frexp's exponent E - 14).  The
           // scales are re-read from vs8 where P is formed, not held here.
           unsigned mh = 0;
+          if constexpr (NG % 2 == 0) {
 #pragma unroll
-          for (int m = 0; m < NG / 2; ++m) {
-            const int k = (e * NG) / 2 + m;
-            const unsigned wd = vs8[ch][k >> 1][k & 1];
-            mh = max(mh, max(wd & 0xffffu, wd >> 16));
+            for (int m = 0; m < NG / 2; ++m) {
+              const int k = (e * NG) / 2 + m;
+              const unsigned wd = vs8[ch][k >> 1][k & 1];
+              mh = max(mh, max(wd & 0xffffu, wd >> 16));
+            }
+          } else {   // a key's scales do not start on a 32-bit word
+#pragma unroll
+            for (int g = 0; g < NG; ++g)
+              mh = max(mh, (unsigned)__builtin_bit_cast(unsigned short, scale_half(vs8, ch, e, g)));
           }
           ex = live && mh ? (float)((int)((mh >> 10) & 31u) - 14) : 0.f;   // (kExpBias 0)
         }
@@ -1151,7 +1160,7 @@ __global__ __launch_bounds__(64 * NW) void stream_i8_kernel(DecodeParams p) {
       }
     }
 #pragma unroll
-    for (int md = 0; md < MD; ++md) {
+    for (int md = 0; md < MDR; ++md) {
       const int g = NG == 1 ? 0 : (16 * md) / 32;
       o[md] = mfma16x16x32<DD_F16>(widen_i8x8_off(v8[md]), pb[g], o[md]);
     }
@@ -1185,7 +1194,7 @@ __global__ __launch_bounds__(64 * NW) void stream_i8_kernel(DecodeParams p) {
 #pragma unroll
   for (int g = 0; g < NG; ++g) psum[g] = kI8Offset * xor32_sum(xor16_sum(psum[g]));
 #pragma unroll
-  for (int md = 0; md < MD; ++md) o[md] -= psum[NG == 1 ? 0 : (16 * md) / 32];
+  for (int md = 0; md < MDR; ++md) o[md] -= psum[NG == 1 ? 0 : (16 * md) / 32];
 
   stream_epilogue<QT, D, NW>(p, s_ml, (float *)s_ring, o, m_run - kExpBias, lsum, w, lane, b, head0, G, split);
 #endif  // __HIP_DEVICE_COMPILE__

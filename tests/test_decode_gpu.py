@@ -465,3 +465,25 @@ def test_config_c3_int8_full_batch():
     cpu = {k: (v.cpu() if torch.is_tensor(v) else v) for k, v in case.items()}
     expected = oracle_case(cpu, rows=rows)
     check(out, expected, torch.int8, rows=rows)
+
+
+@pytest.mark.parametrize('dim', [96, 160, 192, 224])
+@pytest.mark.parametrize('group', [1, 4, 20])
+@pytest.mark.parametrize('window', [0, 100])
+def test_int8_group32_between_the_layouts(dim, group, window):
+    """Group-32 scales at head sizes below the streamed layout that holds them (odd numbers of scales per
+    row among them), unused pages poisoned, one chunk to several splits."""
+    contexts = [1, 15, 33, 700, 1500]
+    case = paged_decode_case(contexts, 2 * group, 2, dim, torch.float32, seed=dim + group)
+    qk, ks = oracle.quantize_q8(case['cache_k'], 32)
+    qv, vs = oracle.quantize_q8(case['cache_v'], 32)
+    used = torch.zeros(case['capacity'], dtype=torch.bool)
+    used[case['page_table'][case['page_table'] >= 0].long()] = True
+    ks[~used], vs[~used] = float('nan'), float('nan')
+    query = case['query'].to(torch.bfloat16)
+    args = (query, qk, qv, case['positions'], case['slots'])
+    out = kernels.attention(*(t.to(DEV) for t in args), window=window, page_table=case['page_table'].to(DEV),
+                            k_scale=ks.to(DEV), v_scale=vs.to(DEV))
+    exp = oracle.decode_attention(*args, window=window, page_table=case['page_table'], k_scale=ks, v_scale=vs)
+    worst, err = excess(out, exp, 5e-3, out.dtype)
+    assert worst <= 0, f'max abs err {err:.3e}'
