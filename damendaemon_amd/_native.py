@@ -30,6 +30,7 @@ SIGNATURES = {
     'dd_abi_version': [],
     'dd_decode_splits': [_i, _i, ctypes.POINTER(_i)],
     'dd_decode_splits_for': [_i, _i, _i, _i, ctypes.POINTER(_i)],
+    'dd_decode_splits_few': [_i, _i, _i, _i, ctypes.POINTER(_i)],
     'dd_decode_attention': [_p, _i, _p, _p, _i, _p, _p, _i,   # q .. group
                             _p, _p, _p, _i, _i,               # positions, slots, table, rows, width
                             _i, _i, _i, _i, _i, _i64, _i, _f,  # B H KH D page cap window scale

@@ -74,6 +74,28 @@ extern "C" int dd_decode_splits_for(int max_context, int batch_kv, int dim, int 
   return n;
 }
 
+// dd_decode_splits_for with smaller splits for launches of few workgroups.
+// The policies above stop at 256 keys per split; with fewer than
+// DD_DECODE_MIN_WG workgroups at that size, most of the GPU idles while eight
+// waves take two or more 16-key chunks each in turn.  128 keys (one chunk a
+// wave), and 64 where that still makes at most 16 splits to merge.  Measured
+// (split kernel + merge): 4 sequences of up to 1,000 fp32 keys, 2 KV heads of
+// 128: 256 keys 11.4 + 3.8 us, 128 8.7 + 3.5, 64 7.4 + 3.8; one sequence of
+// 3,001 bf16 keys, 4 KV heads, room for 16,384: 8.4 + 3.8, 7.2 + 4.2, 6.8 + 6.1.
+extern "C" int dd_decode_splits_few(int max_context, int batch_kv, int dim, int kv_dtype, int *split_tokens) {
+  int st = 0;
+  const int n = dd_decode_splits_for(max_context, batch_kv, dim, kv_dtype, &st);
+  if (n <= 0) return n;
+  long few = st;
+  if ((long)batch_kv * n < DD_DECODE_MIN_WG && st > 64) {
+    few = dd_cdiv(dd_cdiv(max_context, dd_cdiv(DD_DECODE_MIN_WG, batch_kv)), 64) * 64;
+    const long least = max_context <= 16 * 64 ? 64 : 128;
+    few = few < least ? least : (few < st ? few : st);
+  }
+  if (split_tokens) *split_tokens = (int)few;
+  return (int)dd_cdiv(max_context, few);
+}
+
 static int decode_entry(int phase, const void *q, int q_dtype, const void *k, const void *v, int kv_dtype,
                                    const void *k_scale, const void *v_scale, int group,
                                    const int64_t *positions, const int64_t *slots, const int32_t *page_table,

@@ -17,9 +17,10 @@ from . import _native
 from ._native import DTYPE_CODES, call, ptr
 
 
-def _splits(max_context, batch_kv, dim, kv_dtype):
+def _splits(max_context, batch_kv, dim, kv_dtype, policy='dd_decode_splits_few'):
     """Split count and tokens per split: the library's policy for this head
-    size and page dtype, or a fixed split size from
+    size and page dtype (dd_decode_splits_for under a scratch budget: the one
+    with fewer splits), or a fixed split size from
     DAMENDAEMON_AMD_SPLIT_TOKENS (a multiple of 64; tuning)."""
     forced = os.environ.get('DAMENDAEMON_AMD_SPLIT_TOKENS')
     if forced:
@@ -27,14 +28,14 @@ def _splits(max_context, batch_kv, dim, kv_dtype):
         if tokens <= 0 or tokens % 64:
             raise ValueError('DAMENDAEMON_AMD_SPLIT_TOKENS must be a positive multiple of 64')
         return -(-int(max_context) // tokens), tokens
-    return _policy(int(max_context), int(batch_kv), int(dim), DTYPE_CODES[kv_dtype])
+    return _policy(policy, int(max_context), int(batch_kv), int(dim), DTYPE_CODES[kv_dtype])
 
 
 @lru_cache(maxsize=1024)
-def _policy(max_context, batch_kv, dim, kv_code):
+def _policy(name, max_context, batch_kv, dim, kv_code):
     """The library's split policy, a pure function of these numbers."""
     tokens = ctypes.c_int(0)
-    splits = _native.library().dd_decode_splits_for(max_context, batch_kv, dim, kv_code, ctypes.byref(tokens))
+    splits = _native.status(name, max_context, batch_kv, dim, kv_code, ctypes.byref(tokens))
     if splits <= 0:
         raise ValueError('invalid decode geometry')
     return splits, tokens.value
@@ -55,11 +56,13 @@ def attention(query, cache_k, cache_v, positions, slots=None, window=0, scale=No
     damendaemon/kv_quant.py:48-64 generalised to any group that is a
     multiple of 32 or the whole head.
     """
+    policy = 'dd_decode_splits_few'
     if scratch_bytes is not None:
         from .attention_budget import query_rows
+        policy = 'dd_decode_splits_for'
         batch, heads, _, dim = query.shape
         context = cache_k.shape[2] * (1 if page_table is None else page_table.shape[1])
-        splits, _ = _splits(context, batch * cache_k.shape[1], dim, cache_k.dtype)
+        splits, _ = _splits(context, batch * cache_k.shape[1], dim, cache_k.dtype, policy)
         rows = query_rows(heads, dim, splits, scratch_bytes, query.element_size())
         if batch > rows:
             # Partition only independent query rows (kernels.py:237-252); each
@@ -67,15 +70,13 @@ def attention(query, cache_k, cache_v, positions, slots=None, window=0, scale=No
             out = torch.empty_like(query)
             for start in range(0, batch, rows):
                 end = min(start + rows, batch)
-                out[start:end].copy_(attention(
+                out[start:end].copy_(_prepare(
                     query[start:end], cache_k, cache_v, positions[start:end],
-                    None if slots is None else slots[start:end], window=window, scale=scale,
-                    alibi=alibi, page_table=page_table, relative_bias=relative_bias,
-                    relative_max_distance=relative_max_distance, sinks=sinks,
-                    k_scale=k_scale, v_scale=v_scale))
+                    None if slots is None else slots[start:end], window, scale, alibi, page_table, relative_bias,
+                    relative_max_distance, sinks, k_scale, v_scale, None, policy).run())
             return out
-    return prepare_attention(query, cache_k, cache_v, positions, slots, window, scale, alibi, page_table,
-                             relative_bias, relative_max_distance, sinks, k_scale=k_scale, v_scale=v_scale).run()
+    return _prepare(query, cache_k, cache_v, positions, slots, window, scale, alibi, page_table, relative_bias,
+                    relative_max_distance, sinks, k_scale, v_scale, None, policy).run()
 
 
 def prepare_attention(query, cache_k, cache_v, positions, slots=None, window=0, scale=None, alibi=None,
@@ -87,6 +88,12 @@ def prepare_attention(query, cache_k, cache_v, positions, slots=None, window=0, 
 
     Arguments and errors are those of ``attention`` (damendaemon/kernels.py:213-229).
     """
+    return _prepare(query, cache_k, cache_v, positions, slots, window, scale, alibi, page_table, relative_bias,
+                    relative_max_distance, sinks, k_scale, v_scale, out, 'dd_decode_splits_few')
+
+
+def _prepare(query, cache_k, cache_v, positions, slots, window, scale, alibi, page_table, relative_bias,
+             relative_max_distance, sinks, k_scale, v_scale, out, policy):
     batch, heads, _, dim = query.shape
     if alibi is not None and (alibi.shape != (heads,) or alibi.dtype != torch.float32
                               or alibi.device != query.device or not alibi.is_contiguous()):
@@ -131,7 +138,7 @@ def prepare_attention(query, cache_k, cache_v, positions, slots=None, window=0, 
         context = page_table.shape[1] * page_size
     else:
         context = page_size
-    splits, split_tokens = _splits(context, batch * kv_heads, dim, cache_k.dtype)
+    splits, split_tokens = _splits(context, batch * kv_heads, dim, cache_k.dtype, policy)
     return DecodeLaunch(query, cache_k, cache_v, positions, slots, page_table, kv_heads, page_size, capacity,
                         group, k_scale, v_scale, window, scale, alibi, relative_bias, buckets,
                         relative_max_distance, sinks, splits, split_tokens, out)

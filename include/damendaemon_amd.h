@@ -69,6 +69,14 @@ int dd_decode_splits(int max_context, int batch_kv, int *split_tokens);
 int dd_decode_splits_for(int max_context, int batch_kv, int dim, int kv_dtype, int *split_tokens);
 
 /*
+ * dd_decode_splits_for, except that a launch with fewer than 512 workgroups
+ * at 256 keys per split takes splits of 128 keys (64 for contexts up to
+ * 1,024): less time where few sequences leave the GPU idle, for more scratch.
+ * Same return values.
+ */
+int dd_decode_splits_few(int max_context, int batch_kv, int dim, int kv_dtype, int *split_tokens);
+
+/*
  * Ragged decode attention, one query row per sequence.
  * Replaces damendaemon/kernels.py:213-267 (`attention` with the `_attention`
  * and `_merge` Triton kernels), paged (page_table != NULL) or slotted.
@@ -95,7 +103,7 @@ int dd_decode_splits_for(int max_context, int batch_kv, int dim, int kv_dtype, i
  *   out        (batch, heads, dim) q_dtype
  *   partial    fp32 (batch*heads, splits, dim)  scratch (unused if splits==1)
  *   lse        fp32 (batch*heads, splits)       scratch (unused if splits==1)
- *   splits, split_tokens  from dd_decode_splits() or dd_decode_splits_for()
+ *   splits, split_tokens  from dd_decode_splits(), _for() or _few()
  */
 int dd_decode_attention(const void *q, int q_dtype, const void *k,
                         const void *v, int kv_dtype, const void *k_scale,

@@ -487,3 +487,23 @@ def test_int8_group32_between_the_layouts(dim, group, window):
     exp = oracle.decode_attention(*args, window=window, page_table=case['page_table'], k_scale=ks, v_scale=vs)
     worst, err = excess(out, exp, 5e-3, out.dtype)
     assert worst <= 0, f'max abs err {err:.3e}'
+
+
+@pytest.mark.parametrize('width,tokens', [(1024, 64), (4096, 128)])
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+def test_small_splits_of_few_sequences(width, tokens, dtype):
+    """Launches of few workgroups take 64- or 128-key splits: contexts at and beside their edges; under a
+    scratch budget the larger splits stay, and what fitted them still does."""
+    heads, kvh, dim = 8, 2, 64
+    contexts = [1, tokens, tokens + 1, 2 * tokens - 1, width]
+    case = paged_decode_case(contexts, heads, kvh, dim, dtype, seed=width, table_width=width // 16, nan_fill=True)
+    d = {k: (v.to(DEV) if torch.is_tensor(v) else v) for k, v in case.items()}
+    args = (d['query'], d['cache_k'], d['cache_v'], d['positions'], d['slots'])
+    assert kernels._splits(width, 5 * kvh, dim, dtype) == (width // tokens, tokens)
+    exp = oracle.decode_attention(case['query'], case['cache_k'], case['cache_v'], case['positions'], case['slots'],
+                             page_table=case['page_table'])
+    budget = heads * (-(-width // 256) * (dim + 1) * 4 + dim * d['query'].element_size())   # one row at 256 keys
+    for kw in ({}, {'scratch_bytes': budget}):
+        out = kernels.attention(*args, page_table=d['page_table'], **kw)
+        worst, err = excess(out, exp, 2e-5 if dtype == torch.float32 else 2e-3, dtype, 1e-5)
+        assert worst <= 0, f'{kw}: max abs err {err:.3e}'
