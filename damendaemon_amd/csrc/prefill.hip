@@ -156,7 +156,7 @@ static int prefill_entry(int phase, const void *q, const void *k, const void *v,
       const int rc = prefill_x3_dispatch(p, dim, max_len, s);
       if (rc != DD_OK) return rc;
     }
-    if (!(phase & 2)) return DD_OK;
+    if (!(phase & 2) || (max_splits <= 1 && prefill_redo_fits(p.G))) return DD_OK;
     a.flags = p.flags;
     a.flag_rows = kX3Cols / p.G;
     a.flag_tiles = (int)dd_cdiv(max_len, a.flag_rows);
@@ -184,7 +184,9 @@ static int prefill_entry(int phase, const void *q, const void *k, const void *v,
     if (dtype == DD_F16) rc = dispatch<DD_F16>(p, dim, max_len, plan_len, s);
   }
   if (rc != DD_OK || !p.flags || !(phase & 2)) return rc;
-  // the items the bf16 kernel flagged, again in fp32 arithmetic
+  // the items the bf16 kernel flagged, again in fp32 arithmetic (unsplit ones
+  // it has recomputed itself)
+  if (p.max_splits <= 1 && geom.cols == 256 && prefill_redo_fits(p.G)) return DD_OK;
   a.flags = flags;
   a.flag_rows = geom.cols / p.G;
   a.flag_tiles = (int)dd_cdiv(max_len, a.flag_rows);

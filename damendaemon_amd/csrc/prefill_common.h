@@ -3,7 +3,7 @@
 // 16-bit output packing and buffer-resource constants.
 #pragma once
 
-#include "common.h"
+#include "prefill_f32_item.h"
 
 // The running max of a column is only moved when a tile's max exceeds it by
 // more than 2^kMaxSlack in the exp2 domain: probabilities then stay <= 2^8
@@ -124,6 +124,41 @@ DD_DEV unsigned pack2(float a, float b) {
     return (unsigned)float_to_bf16_bits(a) | ((unsigned)float_to_bf16_bits(b) << 16);
   } else {
     return (unsigned)float_to_f16_bits(a) | ((unsigned)float_to_f16_bits(b) << 16);
+  }
+}
+
+// A flagged item again, in fp32 arithmetic and in place (LDS: f32_lds<D>()
+// bytes free for it).  The whole workgroup of W = 8 waves calls it; up to 128
+// query heads per KV head (prefill_redo_fits), beyond that the flags are left
+// to prefill_f32_kernel's launch, which costs 4 us of every call to look for
+// them.  (The code beside the hot loop costs the planned kernel about 1 %: 8 x
+// 512 tokens 226.8 us in one launch, 224.8 + 4 in two.)
+constexpr bool prefill_redo_fits(int G) { return G <= 128; }
+template <int DT, int D, int W>
+DD_DEV void prefill_redo(const PrefillParams &p, char *lds, int grp, int r0, int end) {
+  PrefillGenericArgs a{};
+  a.q = p.q;
+  a.k = p.k;
+  a.v = p.v;
+  a.cu = p.cu;
+  a.ctx = p.ctx;
+  a.slots = p.slots;
+  a.table = p.table;
+  a.out = p.out;
+  a.capacity = p.capacity;
+  a.n = p.n;
+  a.heads = p.H;
+  a.kv_heads = p.KH;
+  a.dim = D;
+  a.page = p.page;
+  a.page_shift = p.page_shift;
+  a.table_w = p.table_w;
+  a.table_rows = p.table_rows;
+  a.window = p.window;
+  a.scale_log2 = p.q_sign ? -p.scale_log2 : p.scale_log2;
+  for (int r = r0; r < end; r += 16 * W / p.G) {
+    __syncthreads();   // the previous users' LDS reads are done
+    f32_item<DT, D, W>(a, lds, grp, r, end);
   }
 }
 

@@ -37,8 +37,10 @@
 // that no result depends on that, each work item checks its output at the
 // end: a column whose largest |O| is not finite or is below 2^-12 (where an
 // absolute 2^-25 could exceed 2^-13 of the row) flags the item in p.flags,
-// and the caller's next launch recomputes the flagged items in fp32
-// arithmetic (prefill_f32.hip, 16-bit values widened exactly).  N(0,1)-like
+// and the workgroup recomputes it in fp32 arithmetic (prefill_f32_item.h,
+// 16-bit values widened exactly); items whose keys are split (flagged by the
+// merge) and those of the 256 layout (whose four waves would spill) are
+// recomputed by another launch.  N(0,1)-like
 // data never takes that path.  The softmax denominators are summed
 // (v_dot2_f32_f16, fp32 accumulate) from exactly the fp16 P that the P.V
 // product uses.
@@ -714,6 +716,12 @@ void prefill_pipe_kernel(PrefillParams p) {
       // segment, so that every flag of a group with work is defined
       if (qt == 0)
         for (int t = (len + rows - 1) / rows + tid; t < p.max_tiles; t += NT) p.flags[(long)grp * p.max_tiles + t] = 0;
+      if constexpr (NW == 8) {
+        if (s_flag && prefill_redo_fits(G)) {
+          prefill_redo<DT, DR, NW>(p, s_kv, grp, r0, r0 + rows_here);
+          continue;
+        }
+      }
     }
   }
   // The output goes through LDS so that every store writes whole 16-byte
@@ -726,6 +734,7 @@ void prefill_pipe_kernel(PrefillParams p) {
   lgkm_drain();
   barrier();
   constexpr int ORS = 2 * DR + 16;      // LDS row stride of the output tile
+  static_assert(NW < 8 || f32_lds<DR>() <= (NKS + NVS) * PLANE, "the fp32 re-run fits the K and V rings");
   static_assert(NW * 32 * ORS <= (NKS + NVS) * PLANE, "output tile fits the K and V rings");
   char *otile = (NW * 32 * ORS <= NVS * PLANE ? s_v : s_kv) + w * 32 * ORS;
   if (colok) {

@@ -18,8 +18,8 @@
 // infinite) gives a non-finite result, and parts below 2^-126 are lost, which
 // shows where a whole result is below 2^-100 or the queries are that small (or
 // so large that a key's lost part counts).  Items with such outputs or queries
-// flag themselves, and the next launch of the call recomputes flagged items
-// with fp32 matrix instructions (prefill_f32.hip).
+// flag themselves, and the workgroup recomputes them with fp32 matrix
+// instructions (prefill_f32_item.h; another launch where keys are split).
 //
 // Work split.  Bound by the matrix cores: a workgroup of eight waves (two per
 // SIMD, one workgroup per CU) owns 256 (query row, head) columns of one
@@ -113,8 +113,11 @@ void prefill_x3_kernel(PrefillParams p) {
   constexpr int VPART = 2048 * MD;          // ... of a V tile: (16-key step, dim block, half) regions of 512
   static_assert(KT == 32 && KT * PD <= NT, "one piece per thread");
 
-  __shared__ __align__(16) char s_k[2][3 * KPART];
-  __shared__ __align__(16) char s_v[2][3 * VPART];
+  __shared__ __align__(16) char s_mem[6 * (KPART + VPART)];
+  static_assert(f32_lds<D>() <= 6 * (KPART + VPART), "the fp32 re-run fits");
+  // [2][3 parts] of K, then of V
+  auto s_k = [&](int buf) __attribute__((always_inline)) { return s_mem + buf * 3 * KPART; };
+  auto s_v = [&](int buf) __attribute__((always_inline)) { return s_mem + 6 * KPART + buf * 3 * VPART; };
   __shared__ int s_flag;
 
   const int tid = threadIdx.x;
@@ -192,12 +195,12 @@ void prefill_x3_kernel(PrefillParams p) {
     if (pload) {
       split3(kr, r);
 #pragma unroll
-      for (int j = 0; j < 3; ++j) *(u32x4 *)(s_k[buf] + j * KPART + k_wr) = r[j];
+      for (int j = 0; j < 3; ++j) *(u32x4 *)(s_k(buf) + j * KPART + k_wr) = r[j];
     }
     if (piece) {
       split3(vr, r);
 #pragma unroll
-      for (int j = 0; j < 3; ++j) *(u32x4 *)(s_v[buf] + j * VPART + v_wr) = r[j];
+      for (int j = 0; j < 3; ++j) *(u32x4 *)(s_v(buf) + j * VPART + v_wr) = r[j];
     }
   };
 
@@ -222,7 +225,7 @@ void prefill_x3_kernel(PrefillParams p) {
     for (int c = 0; c < NCC; ++c) {
       u32x4 ka[3];
 #pragma unroll
-      for (int j = 0; j < 3; ++j) ka[j] = *(const u32x4 *)(s_k[buf] + j * KPART + 2 * c * kKBlock + k_rd);
+      for (int j = 0; j < 3; ++j) ka[j] = *(const u32x4 *)(s_k(buf) + j * KPART + 2 * c * kKBlock + k_rd);
       s = mfma_x3(ka, qa[c], s);
     }
     // ---- softmax: register r holds key 32 t + 8 (r / 4) + 4 h2 + r % 4 ----
@@ -275,7 +278,7 @@ void prefill_x3_kernel(PrefillParams p) {
         u32x4 va[3];
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
-          const char *src = s_v[buf] + j * VPART + (j2 * MD + md) * 1024 + 8 * lane;
+          const char *src = s_v(buf) + j * VPART + (j2 * MD + md) * 1024 + 8 * lane;
           const u32x2 lo = lds_tr(src), hi = lds_tr(src + 512);
           va[j] = u32x4{lo[0], lo[1], hi[0], hi[1]};
         }
@@ -324,6 +327,10 @@ void prefill_x3_kernel(PrefillParams p) {
   if (it.qt == 0)
     for (int t = (it.len + rows - 1) / rows + tid; t < p.max_tiles; t += NT)
       p.flags[(long)it.grp * p.max_tiles + t] = 0;
+  if (s_flag && prefill_redo_fits(G)) {
+    prefill_redo<DD_F32, D, kX3Waves>(p, s_mem, it.grp, r0, r0 + rows_here);
+    return;
+  }
   if (!colok) return;
   const float inv = 1.f / l;
 #pragma unroll

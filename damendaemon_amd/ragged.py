@@ -172,8 +172,9 @@ class PrefillLaunch:
         return self.phase(3)
 
     def phase(self, which):
-        """Enqueue one launch of the call: 1 the attention kernel, 2 the exact
-        re-run of the items the bf16 kernel flagged (both together = run())."""
+        """Enqueue one phase of the call: 1 the attention kernel (and the merge
+        of split items), 2 the exact re-run of flagged items that it did not
+        recompute itself (both together = run())."""
         if self._args is not None:
             call('dd_prefill_attention_split', *self._args, int(which), _native.stream_on(self._index))
         return self.out

@@ -316,10 +316,11 @@ int dd_prefill_attention(const void *q, const void *k, const void *v,
                          void *out, void *stream);
 
 /*
- * dd_prefill_attention in two launches (same arguments): phase 1 runs the
- * attention kernel, phase 2 the exact re-run of the work items the bf16
- * kernel flagged (a no-op for calls without a flags workspace); 3 = both,
- * as dd_prefill_attention.  For timing the attention kernel on its own.
+ * dd_prefill_attention in two phases (same arguments): phase 1 runs the
+ * attention kernel (and the merge of split items), phase 2 the exact re-run
+ * of the work items it flagged and could not recompute itself: split ones,
+ * head sizes above 160, more than 128 query heads per KV head (a no-op for
+ * other calls); 3 = both, as dd_prefill_attention.  For timing the attention kernel on its own.
  */
 int dd_prefill_attention_phase(const void *q, const void *k, const void *v,
                                int dtype, const int64_t *cu_seqlens,
